@@ -768,40 +768,156 @@ __global__ __launch_bounds__(kGThreads, 1) void gqa_decode_wide_kernel(
   }
 }
 
-// LSE combine of the split partials of one query row per wave:
+// LSE combine of the split partials of a query row:
 // lse = logsumexp_s lse_s, out = sum_s exp(lse_s - lse) o_s.
-template <typename T>
+//
+// Bound by the latency of its loads, not by their bytes, so a row's splits are spread over
+// the lanes: kTeam threads per row, D / 4 lanes (4 dims each) per split, kPar splits side
+// by side and kBatch of each lane's splits requested at once, their lse beside their
+// values.  Every lane folds its splits against its own running max, and the lanes of one
+// dim group are merged at the end (shuffles inside a wave, LDS between waves).  One wave per
+// row covers up to kWaveSplits splits; above that four waves do (a long context over few rows
+// has too few rows to fill the chip).  A wave that walked the splits one after the other
+// took 18.7 us for 16 splits of 32 rows at D = 128, against 4.8 us (kernel trace), and
+// 6.7 us for 4 splits of 256 rows, against 3.8 us.
+constexpr int kWaveSplits = 16;
+
+template <typename T, int D, int kTeam>
 __global__ __launch_bounds__(256) void gqa_combine_kernel(const fa_gqa_decode_args a) {
-  const long long row = static_cast<long long>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  typedef typename Vec<T>::v4 T4;
+  constexpr int kLanes = D / 4 < kTeam ? D / 4 : kTeam;  // lanes per split
+  constexpr int kVec = D / 4 / kLanes;                   // 4-dim pieces per lane
+  constexpr int kPar = kTeam / kLanes;                   // splits side by side
+  constexpr int kBatch = kTeam == 64 ? 4 : 8;
+  constexpr int kGroups = kLanes > 64 ? kPar : kTeam / 64;  // states left after the shuffles
+  __shared__ floatx4 sacc[kGroups > 1 ? kGroups * (D / 4) : 1];
+  __shared__ float sml[kGroups > 1 ? 2 * kGroups : 1];
+  const long long row = static_cast<long long>(blockIdx.x) * (256 / kTeam) + threadIdx.x / kTeam;
   const long long nrows = static_cast<long long>(a.batch) * a.h_q * a.m;
-  if (row >= nrows) return;
-  const int lane = threadIdx.x & 63;
+  if (row >= nrows) return;  // whole waves; whole work-groups where there is a barrier
+  const int tid = threadIdx.x % kTeam;
+  const int sub = tid / kLanes, d4 = tid % kLanes;
   const int S = a.num_splits;
   const float ninf = -__builtin_inff();
-  const float* lp = a.lse_part + row * S;
-  float mx = ninf;
-  for (int s = lane; s < S; s += 64) mx = fmaxf(mx, lp[s]);
-  for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-  float sum = 0.f;
-  if (mx != ninf)
-    for (int s = lane; s < S; s += 64) sum += expf(lp[s] - mx);
-  for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
-  const float lse = sum > 0.f ? mx + logf(sum) : ninf;
-  const int D = a.d;
+  const float* const lp = a.lse_part + row * S;
+  const float* const op = a.o_part + row * S * D + 4 * d4;
+  float m = ninf, l = 0.f;
+  floatx4 acc[kVec];
+#pragma unroll
+  for (int v = 0; v < kVec; ++v) acc[v] = floatx4{};
+  for (int s0 = sub; s0 < S; s0 += kPar * kBatch) {
+    float lv[kBatch];
+    floatx4 ov[kBatch][kVec];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int s = min(s0 + kPar * i, S - 1);
+      lv[i] = lp[s];
+#pragma unroll
+      for (int v = 0; v < kVec; ++v)
+        ov[i][v] = *reinterpret_cast<const floatx4*>(op + static_cast<long long>(s) * D +
+                                                     4 * kLanes * v);
+    }
+    float mb = m;
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      if (s0 + kPar * i >= S) lv[i] = ninf;
+      mb = fmaxf(mb, lv[i]);
+    }
+    if (mb == ninf) continue;
+    const float f = m == ninf ? 0.f : expf(m - mb);
+    m = mb;
+    l *= f;
+#pragma unroll
+    for (int v = 0; v < kVec; ++v)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) acc[v][x] *= f;
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      if (lv[i] == ninf) continue;  // an empty split's values are not read
+      const float w = expf(lv[i] - mb);
+      l += w;
+#pragma unroll
+      for (int v = 0; v < kVec; ++v)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) acc[v][x] += w * ov[i][v][x];
+    }
+  }
+  // merge the states of one dim group inside the wave
+#pragma unroll
+  for (int off = 32; off >= kLanes; off >>= 1) {
+    const float m2 = __shfl_xor(m, off), l2 = __shfl_xor(l, off);
+    const float mn = fmaxf(m, m2);
+    const float f1 = m == ninf ? 0.f : expf(m - mn), f2 = m2 == ninf ? 0.f : expf(m2 - mn);
+    m = mn;
+    l = l * f1 + l2 * f2;
+#pragma unroll
+    for (int v = 0; v < kVec; ++v)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const float o2 = __shfl_xor(acc[v][x], off);
+        acc[v][x] = acc[v][x] * f1 + o2 * f2;
+      }
+  }
+  if constexpr (kGroups > 1) {  // kTeam = 256, one row per work-group, kVec = 1
+    constexpr int kGroupThreads = kTeam / kGroups;
+    const int grp = tid / kGroupThreads;
+    if (tid % kGroupThreads < kLanes) {
+      sacc[grp * (D / 4) + d4] = acc[0];
+      if (d4 == 0) {
+        sml[2 * grp] = m;
+        sml[2 * grp + 1] = l;
+      }
+    }
+    __syncthreads();
+    if (tid >= D / 4) return;
+    m = ninf;
+#pragma unroll
+    for (int i = 0; i < kGroups; ++i) m = fmaxf(m, sml[2 * i]);
+    l = 0.f;
+    acc[0] = floatx4{};
+#pragma unroll
+    for (int i = 0; i < kGroups; ++i) {
+      const float f = sml[2 * i] == ninf ? 0.f : expf(sml[2 * i] - m);
+      l += f * sml[2 * i + 1];
+      const floatx4 o = sacc[i * (D / 4) + tid];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) acc[0][x] += f * o[x];
+    }
+  } else if (sub != 0) {
+    return;
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
   const long long b = row / (static_cast<long long>(a.h_q) * a.m);
   const long long hm = row - b * a.h_q * a.m;
-  const int h = static_cast<int>(hm / a.m), mq = static_cast<int>(hm - h * a.m);
-  T* op = static_cast<T*>(a.out) + b * a.o_stride_b + h * a.o_stride_h + mq * a.o_stride_m;
-  for (int d = lane; d < D; d += 64) {
-    float o = 0.f;
-    if (lse != ninf)
-      for (int s = 0; s < S; ++s) {
-        const float ls = lp[s];
-        if (ls != ninf) o += expf(ls - lse) * a.o_part[(row * S + s) * D + d];
-      }
-    op[d] = static_cast<T>(o);
+  const int h = static_cast<int>(hm / a.m), mq = static_cast<int>(hm - static_cast<long long>(h) * a.m);
+  T* const out = static_cast<T*>(a.out) + b * a.o_stride_b + h * a.o_stride_h +
+                 mq * a.o_stride_m + 4 * d4;
+  const bool wide = ((reinterpret_cast<uintptr_t>(a.out) & 7) | (a.o_stride_b & 3) |
+                     (a.o_stride_h & 3) | (a.o_stride_m & 3)) == 0;  // uniform
+#pragma unroll
+  for (int v = 0; v < kVec; ++v) {
+    T4 w;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) w[x] = static_cast<T>(acc[v][x] * inv);
+    if (wide) {
+      *reinterpret_cast<T4*>(out + 4 * kLanes * v) = w;
+    } else {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) out[4 * kLanes * v + x] = w[x];
+    }
   }
-  if (lane == 0 && a.lse) a.lse[row] = lse;
+  if (tid == 0 && a.lse) a.lse[row] = l > 0.f ? m + logf(l) : ninf;
+}
+
+template <typename T, int D>
+void launch_combine(const fa_gqa_decode_args* a, hipStream_t stream) {
+  const long long rows = static_cast<long long>(a->batch) * a->h_q * a->m;
+  if (a->num_splits <= kWaveSplits)
+    hipLaunchKernelGGL((gqa_combine_kernel<T, D, 64>), dim3(static_cast<unsigned>((rows + 3) / 4)),
+                       dim3(256), 0, stream, *a);
+  else
+    hipLaunchKernelGGL((gqa_combine_kernel<T, D, 256>), dim3(static_cast<unsigned>(rows)),
+                       dim3(256), 0, stream, *a);
 }
 
 template <typename T, bool kPaged>
@@ -886,13 +1002,23 @@ extern "C" int fa_gqa_combine(const fa_gqa_decode_args* a, void* stream) {
   int rc = fa::check_gqa(a);
   if (rc != FA_OK) return rc;
   FA_CHECK_ARG(a->o_part && a->lse_part, "combine needs o_part and lse_part");
-  const long long rows = static_cast<long long>(a->batch) * a->h_q * a->m;
-  const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (a->dtype == 1)
-    hipLaunchKernelGGL(fa::gqa_combine_kernel<__bf16>, grid, dim3(256), 0, s, *a);
-  else
-    hipLaunchKernelGGL(fa::gqa_combine_kernel<_Float16>, grid, dim3(256), 0, s, *a);
+  switch (a->d) {
+#define FA_COMBINE_CASE(DD)                          \
+  case DD:                                           \
+    if (a->dtype == 1)                               \
+      fa::launch_combine<__bf16, DD>(a, s);          \
+    else                                             \
+      fa::launch_combine<_Float16, DD>(a, s);        \
+    break;
+    FA_COMBINE_CASE(16)
+    FA_COMBINE_CASE(32)
+    FA_COMBINE_CASE(64)
+    FA_COMBINE_CASE(128)
+    FA_COMBINE_CASE(256)
+    FA_COMBINE_CASE(512)
+#undef FA_COMBINE_CASE
+  }
   FA_CHECK_HIP(hipGetLastError());
   return FA_OK;
 }

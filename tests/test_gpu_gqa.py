@@ -335,3 +335,11 @@ def test_paged_attention_split_longer_than_lds_table(head_size):
     split's block-table slice does not fit in LDS and the pages are looked up in global
     memory (the other loop of both kernels)."""
     base_paged_attention(2, 4, 1, head_size, 8, 20000, 1, seed=head_size)
+
+
+@pytest.mark.parametrize("head_size", [16, 64, 128, 256, 512])
+@pytest.mark.parametrize("num_splits", [16, 32, 128])
+def test_paged_attention_many_splits(head_size, num_splits):
+    """The combine on both sides of its team size (one wave per row up to 16 splits, four
+    above) with splits past the end of the short sequences (empty partials)."""
+    base_paged_attention(3, 4, 2, head_size, 16, 4096, num_splits, seed=head_size + num_splits)
