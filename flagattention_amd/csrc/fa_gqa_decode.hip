@@ -38,6 +38,7 @@
 // gather, masking, online softmax, per-split (o, lse) -- and the LSE combine
 // of _fwd_combine_kv_splits (src/flag_attn/split_kv.py:176-241).
 #include "fa_common.h"
+#include "fa_prefill.h"
 #include "fa_wave.h"
 
 namespace fa {
@@ -991,6 +992,7 @@ extern "C" int fa_gqa_decode(const fa_gqa_decode_args* a, void* stream) {
   if (rc != FA_OK) return rc;
   FA_CHECK_ARG(a->num_splits == 1 || (a->o_part && a->lse_part),
                "num_splits %d > 1 needs o_part and lse_part", a->num_splits);
+  if (fa::prefill_takes(a)) return fa::launch_prefill(a, stream);
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const bool paged = a->block_table != nullptr;
   if (a->dtype == 1)

@@ -36,6 +36,15 @@ from .errors import ArgumentError
 HEAD_DIMS = (16, 32, 64, 128, 256, 512)
 ROWS_PER_WG = 16
 MIN_SPLIT_TOKENS = 256
+# The many-row kernel (csrc/fa_prefill.h): head dims, rows per KV head above which the
+# library uses it for contiguous K/V, and its rows per work-group.
+PREFILL_DIMS = (64, 128, 256)
+PREFILL_MIN_ROWS = 16
+PREFILL_ROWS_PER_WG = 128
+# Up to here the second launch costs more than the keys it saves a work-group: a 300-token
+# prompt (8 KV heads, D = 128) takes 18.7 us unsplit, 25.4 us in two splits; at 2,000 keys
+# (D = 256, 4 KV heads) 8 splits take 27.9 us, 4 of them 36.4 us.
+PREFILL_UNSPLIT_TOKENS = 512
 
 # Benchmark hook: a (start, end) pair of CUDA events recorded on the launch stream right
 # around the next decode kernel launch (not the combine); cleared after that launch.
@@ -67,11 +76,11 @@ def _cu_count(device: torch.device) -> int:
 
 
 def choose_splits(batch: int, h_kv: int, rows_per_kv_head: int, max_len: int,
-                  cu_count: int) -> int:
+                  cu_count: int, rows_per_wg: int = ROWS_PER_WG) -> int:
     """Split-KV count: none when batch x KV heads x row blocks already gives every CU a
     work-group, else enough splits for about two work-groups per CU, each at least
     MIN_SPLIT_TOKENS keys long."""
-    base = batch * h_kv * -(-rows_per_kv_head // ROWS_PER_WG)
+    base = batch * h_kv * -(-rows_per_kv_head // rows_per_wg)
     if base >= cu_count or max_len <= MIN_SPLIT_TOKENS:
         return 1
     return max(1, min(-(-2 * cu_count // base), -(-max_len // MIN_SPLIT_TOKENS)))
@@ -196,7 +205,11 @@ def _dense_decode(q, k, v, causal, sm_scale, want_lse):
     if o.stride(-1) != 1 or not _aligned(o, (0, 1, 2)):
         o = torch.empty(q.shape, dtype=q.dtype, device=device)
     lse = torch.empty((batch, h_q, m), dtype=torch.float32, device=device) if want_lse else None
-    s = choose_splits(batch, h_kv, (h_q // h_kv) * m, n, _cu_count(device))
+    rows = (h_q // h_kv) * m
+    many = d in PREFILL_DIMS and rows > PREFILL_MIN_ROWS
+    s = (1 if many and n <= PREFILL_UNSPLIT_TOKENS
+         else choose_splits(batch, h_kv, rows, n, _cu_count(device),
+                            PREFILL_ROWS_PER_WG if many else ROWS_PER_WG))
     split_tokens = -(-n // s) if n > 0 else 1
     s = max(1, -(-n // split_tokens)) if n > 0 else 1
     if s == 1:

@@ -290,7 +290,10 @@ int64_t fa_gqa_decode_args_size(void);
 /*
  * Decode: with num_splits == 1 writes out (and lse if given); otherwise the
  * per-split partials (o_part normalised per split, lse_part) for
- * fa_gqa_combine.  Head dims 16, 32, 64, 128, 256, 512.
+ * fa_gqa_combine.  Head dims 16, 32, 64, 128, 256, 512.  Contiguous K/V with more
+ * than 16 query rows per KV head (group x m) at head dims 64, 128, 256 runs the
+ * 128-row kernel of fa_prefill.hip (out must then have 16-byte aligned rows; if not,
+ * the 16-row kernel runs).
  * Replaces _paged_attn_kernel, src/flag_attn/paged.py:218-363 (paged) and
  * _fwd_split_kv_kernel, src/flag_attn/split_kv.py:28-174 (contiguous).
  */

@@ -343,3 +343,65 @@ def test_paged_attention_many_splits(head_size, num_splits):
     """The combine on both sides of its team size (one wave per row up to 16 splits, four
     above) with splits past the end of the short sequences (empty partials)."""
     base_paged_attention(3, 4, 2, head_size, 16, 4096, num_splits, seed=head_size + num_splits)
+
+
+def _laid_out(x, form):
+    """The values of [B, H, T, D] tensor x in another memory layout."""
+    b, h, t, d = x.shape
+    if form == "bhtd":
+        return x.to(DEV).contiguous()
+    if form == "bthd":
+        return x.to(DEV).transpose(1, 2).contiguous().transpose(1, 2)
+    if form == "padded":  # rows of a wider buffer
+        wide = torch.zeros((b, h, t + 3, d + 8), dtype=x.dtype, device=DEV)
+        wide[:, :, :t, :d] = x.to(DEV)
+        return wide[:, :, :t, :d]
+    wide = torch.zeros((b, h, t, d + 1), dtype=x.dtype, device=DEV)  # "odd": rows not 16-aligned
+    wide[..., 1:] = x.to(DEV)
+    return wide[..., 1:]
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("B, Hq, Hk, M, N, causal, form", [
+    (1, 2, 2, 17, 1, False, "bhtd"),      # the fewest rows, one key
+    (2, 6, 2, 43, 65, True, "bthd"),      # 129 rows: a second work-group with one row
+    (1, 8, 1, 16, 64, True, "padded"),    # 128 rows, one whole tile
+    (1, 3, 1, 11, 63, True, "bhtd"),      # 33 rows: a second wave with one row
+    (2, 4, 4, 127, 127, True, "odd"),     # realigned by a copy, short of a tile
+    (8, 16, 8, 300, 193, True, "bthd"),   # M > N, every work-group resident at once
+    (1, 4, 2, 40, 2100, True, "padded"),  # splits, the last one ragged
+    (3, 3, 1, 200, 1600, False, "bhtd"),  # a batch that is not a multiple of the XCDs
+])
+def test_flash_attention_many_rows(D, B, Hq, Hk, M, N, causal, form):
+    """More than 16 query rows per KV head (128 per work-group, 32 per wave, 32- or 64-key
+    tiles): edges of rows, tiles and splits, each layout, both dtypes, both signs of the
+    scale.  Same rule and lse bar as the other contiguous decodes."""
+    need_gpu()
+    for dtype, scale in ((torch.float16, D ** -0.5), (torch.bfloat16, -D ** -0.5)):
+        q, k, v = _splitkv_inputs(B, Hq, Hk, M, N, D, dtype, "BHTD", 1.0, D + M + N)
+        o_ref, lse_ref = go.flash_attention_ref(q, k, v, causal, sm_scale=scale, upcast=True)
+        o_low, _ = go.flash_attention_ref(q, k, v, causal, sm_scale=scale, upcast=False)
+        o, lse, _, _, _ = flag_attn.flash_attention(
+            *(_laid_out(x, form) for x in (q, k, v)), causal, scale, return_log_normalizer=True)
+        torch.cuda.synchronize()
+        o, lse = o.cpu(), lse.cpu()
+        assert bool(torch.isfinite(o).all())
+        assert_lowp_rule(o, o_ref, o_low)
+        assert torch.equal(torch.isneginf(lse), torch.isneginf(lse_ref))
+        fin = ~torch.isneginf(lse_ref)
+        assert float((lse[fin] - lse_ref[fin]).abs().max()) <= 1e-3
+
+
+def test_flash_attention_many_rows_late_maximum():
+    """Scores that keep growing along the keys (each tile's maximum far above the one before):
+    the accumulators are rescaled at every tile, and no probability overflows fp16."""
+    need_gpu()
+    q, k, v = _splitkv_inputs(1, 2, 1, 40, 700, 64, torch.float16, "BHTD", 1.0, 5)
+    q[..., 0], k[..., 0] = 8.0, torch.arange(700, dtype=torch.float16) / 16
+    o_ref, lse_ref = go.flash_attention_ref(q, k, v, False, upcast=True)
+    o_low, _ = go.flash_attention_ref(q, k, v, False, upcast=False)
+    o, lse, _, _, _ = flag_attn.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), False,
+                                                return_log_normalizer=True)
+    torch.cuda.synchronize()
+    assert_lowp_rule(o.cpu(), o_ref, o_low)
+    assert float((lse.cpu() - lse_ref).abs().max()) <= 1e-3
