@@ -167,7 +167,8 @@ def algorithmic_work(spec, lens_cpu, indices) -> tuple:
 # it includes); a traffic record holds only while these are unchanged.
 _SHARED = ("flagattention_amd/csrc/fa_common.h", "flagattention_amd/csrc/fa_wave.h",
            "include/flagattention_amd.h")
-DECODE_SOURCES = ("flagattention_amd/csrc/fa_decode.hip",) + _SHARED
+DECODE_SOURCES = ("flagattention_amd/csrc/fa_decode.hip",
+                  "flagattention_amd/csrc/fa_mla_tile.h") + _SHARED
 KERNEL_SOURCES = {
     "mla_decode": DECODE_SOURCES,
     "gqa_decode": ("flagattention_amd/csrc/fa_gqa_decode.hip",) + _SHARED,

@@ -62,27 +62,16 @@
 #include <utility>
 
 #include "fa_common.h"
+#include "fa_mla_tile.h"
 #include "fa_wave.h"
 
 namespace fa {
 namespace {
 
-constexpr int kThreads = 256;                    // 4 waves, one per SIMD
-constexpr int kTileRows = 32;                    // tokens per pipeline tile
-constexpr int kRowBytes = kDqk * 2;              // 1152 B: one bf16 cache row
-constexpr int kChunkGroups = kRowBytes / 128;    // 9 groups of 8 chunks per row
-constexpr int kBlockBytes = 1024;                // 8 rows x 8 chunks
-constexpr int kRowGroupBytes = kChunkGroups * kBlockBytes;  // 9216
-constexpr int kTileBytes = kTileRows * kRowBytes;  // 36864 B per LDS tile
-constexpr int kFp8RowBytes = FA_MLA_FP8_ROW_BYTES;  // 656
-constexpr int kQkSteps = kDqk / 32;              // 18 MFMA k-steps of QK
 constexpr int kDimTiles = kDv / 4 / 16;          // 8 16-dim tiles of O^T per wave
 constexpr int kRowTiles = kRows / 16;            // 8 16-row tiles
-constexpr int kCopiesPerWave = kChunkGroups;     // 9 wave-wide copies per tile
 constexpr int kQOps = 2 * kQkSteps;              // 36 Q^T operands (k-step, row tile) per wave
 constexpr int kQLds = 4;                          // sparse: the first ones live in LDS, not VGPRs
-
-enum Mode { kDense = 0, kSparseBf16 = 1, kSparseFp8 = 2 };
 
 // Shared state beside the three tile buffers (separate LDS objects, see the
 // kernel, so the compiler can prove that reads of one never alias a copy
@@ -173,90 +162,6 @@ __device__ inline void copy_block_buf(__amdgpu_buffer_rsrc_t rs, unsigned char* 
   constexpr int kNonTemporal = 2;  // CPol NT
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (FA_LDS void*)(dst + G * (kBlockBytes - 128)), 16,
                                            voff, 0, 128 * G, kNonTemporal);
-}
-
-// fp8-e4m3 (OCP "fn") pair -> two floats, using the gfx950 converter.
-template <bool kHi>
-__device__ inline floatx2 fp8x2_to_f32(unsigned int word) {
-  return __builtin_amdgcn_cvt_pk_f32_fp8(word, kHi);
-}
-
-__device__ inline unsigned int pack_bf16x2(float a, float b) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  floatx2 f;
-  f[0] = a;
-  f[1] = b;
-  return __builtin_bit_cast(unsigned int, __builtin_convertvector(f, bf16x2));  // one v_cvt_pk_bf16_f32
-}
-
-// fp8 tiles reach LDS raw, one row-group (8 tile rows) per wave, inside the
-// row-group's own 9 KB of the bf16 tile buffer:
-//   [0, 4096)      codes: block G (1 KB) holds codes 128G..128G+127 of the 8
-//                  rows, slot 8r + c = row r, 16-byte chunk c
-//   [4096, 5120)   the four fp32 scales of row r at 4096 + 128r (the copy
-//                  lanes of a row all load them; slot 8r is the one read)
-//   [8192, 9216)   the rope dims, already in the bf16 layout (chunk-group 8)
-// and the wave that loaded them turns the codes into bf16 blocks 0..7 in
-// place.  Those overlap the raw bytes, so every read of the row-group comes
-// before its first write; no other wave touches the row-group meanwhile.
-constexpr int kFp8Copies = 6;          // wave-wide 16-byte copies per row-group
-constexpr int kFp8ScaleOff = 4096;
-
-// The conversion in two parts, so that a step can spread it over its MFMAs:
-// fp8_load reads this lane's 64 codes and their scale (all the row-group's
-// reads, before any write), fp8_store<I, H> converts and writes one 16-byte
-// bf16 chunk of them (8 calls cover the lane).  Addresses are rebuilt from a
-// fresh lane id: kept live across the loop they would be spilled, and each
-// reload would stall the conversion.
-struct Fp8Codes {
-  uintx4 code[4];
-  float scale;
-  int base;  // byte offset of the lane's row r, chunk-group e in the row-group
-  int r;     // row of the lane in the row-group (the chunk swizzle)
-  int eh;    // e / 2: the lane's rotation of its four pieces
-};
-__device__ inline Fp8Codes fp8_load(const unsigned char* buf, int wave) {
-  const int lane = fresh_lane();
-  const int r = lane >> 3, e = lane & 7;  // row r of the group, codes 64e..64e+63
-  const unsigned char* rg = buf + wave * kRowGroupBytes;
-  const unsigned char* src = rg + 1024 * (e >> 1) + 16 * (8 * r + 4 * (e & 1));
-  // Lane (r, e) takes its four 16-code pieces in the order m = (i + e/2) % 4: the
-  // reads of one instruction then fall in 16 different bank groups per 16 lanes, and
-  // its writes in 8 (2-way) instead of 2 (8-way).
-  const int rot = e >> 1;
-  Fp8Codes c;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    c.code[i] = *reinterpret_cast<const uintx4*>(src + 16 * ((i + rot) & 3));
-  c.scale = *reinterpret_cast<const float*>(rg + kFp8ScaleOff + 128 * r + 4 * (e >> 1));
-  c.base = (kChunkGroups * wave + e) * kBlockBytes + 128 * r;  // tile_off(8 wave + r, 8 e)
-  c.r = r;
-  c.eh = rot;
-  return c;
-}
-// Byte offset of piece I, half H of the lane: tile_off(8 wave + r, 8 e + 2 m + H).
-template <int I, int H>
-__device__ inline int fp8_store_off(const Fp8Codes& c) {
-  return c.base + 16 * ((2 * ((I + c.eh) & 3) + H) ^ c.r);
-}
-template <int I, int H>  // piece I of the four, half H: 8 codes -> one 16-byte bf16 chunk
-__device__ inline void fp8_store(unsigned char* buf, const Fp8Codes& c) {
-  const unsigned int w0 = c.code[I][2 * H], w1 = c.code[I][2 * H + 1];
-  floatx2 a = fp8x2_to_f32<false>(w0), b = fp8x2_to_f32<true>(w0);
-  floatx2 d = fp8x2_to_f32<false>(w1), f = fp8x2_to_f32<true>(w1);
-  uintx4 o;
-  o[0] = pack_bf16x2(a[0] * c.scale, a[1] * c.scale);
-  o[1] = pack_bf16x2(b[0] * c.scale, b[1] * c.scale);
-  o[2] = pack_bf16x2(d[0] * c.scale, d[1] * c.scale);
-  o[3] = pack_bf16x2(f[0] * c.scale, f[1] * c.scale);
-  *reinterpret_cast<uintx4*>(buf + fp8_store_off<I, H>(c)) = o;
-}
-__device__ inline void dequant_fp8_rowgroup(unsigned char* buf, int wave) {
-  const Fp8Codes c = fp8_load(buf, wave);
-  static_for<8>([&](auto pt) {
-    constexpr int P = decltype(pt)::value;
-    fp8_store<P / 2, P % 2>(buf, c);
-  });
 }
 
 template <int kMode>
@@ -1210,6 +1115,9 @@ int launch_decode(const fa_mla_decode_args* a, hipStream_t stream) {
   // dense: flattened (s, h) rows; sparse: one query token per work-group
   const int num_m_blocks = kMode == kDense ? cdiv(a->s_q * a->h_q, kRows)
                                            : a->s_q * cdiv(a->h_q, kRows);
+  // rows that share one KV stream: few of them leave the 128-row kernel mostly idle
+  if ((kMode == kDense ? static_cast<long long>(a->s_q) * a->h_q : a->h_q) <= kFewRowsMax)
+    return launch_decode_few(a, kMode, stream);
   const int grid = a->num_parts * num_m_blocks;
   hipLaunchKernelGGL(mla_decode_kernel<kMode>, dim3(grid), dim3(kThreads), 0, stream, *a,
                      num_m_blocks);
