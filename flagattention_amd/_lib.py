@@ -11,6 +11,7 @@ import threading
 
 ABI_VERSION = 3
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libflagattention_amd.so")
+NATIVE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_native.so")
 
 FA_OK = 0
 
@@ -169,6 +170,30 @@ def load() -> ctypes.CDLL:
                 f"{ctypes.sizeof(GqaArgs)} in the binding")
         _lib = lib
         return lib
+
+
+_native = None  # the host module once loaded
+
+
+def native():
+    """The native host path (csrc/host/fa_native.cpp), loaded once: functions that run a usual
+    call whole and return None for any other, which the Python path then handles.  None if
+    nothing is built (the Python path then raises); a library without it raises."""
+    global _native
+    if _native is None:
+        if not os.path.exists(LIB_PATH):
+            return None
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(
+                f"flagattention_amd: host module not found at {NATIVE_PATH}; "
+                "build it with `python -m flagattention_amd.build`")
+        load()
+        from . import _native as mod
+        if mod.ABI_VERSION != ABI_VERSION:
+            raise RuntimeError(
+                f"flagattention_amd: host module ABI {mod.ABI_VERSION} != {ABI_VERSION}")
+        _native = mod
+    return _native
 
 
 def check(rc: int) -> None:

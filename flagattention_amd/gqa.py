@@ -127,6 +127,12 @@ def paged_attention(
     ``block_tables[s, j // block_size]`` (``testing/paged.py:44-47``); a page id outside the
     cache reads as a masked key.  Returns ``out`` shaped and typed like ``query``.
     """
+    fast = _lib.native() if timing_events is None else None
+    if fast is not None:
+        done = fast.paged(query, key_cache, value_cache, context_lens, block_tables, attn_scale,
+                          max_context_len, num_splits)
+        if done is not None:
+            return done
     _require(query.dim() == 3, "query must be [num_seqs, num_heads, head_size]")
     _require(key_cache.dim() == 4 and value_cache.shape == key_cache.shape,
              "key_cache / value_cache must be [num_blocks, num_kv_heads, block_size, head_size]")
@@ -182,6 +188,11 @@ def paged_attention(
 
 
 def _dense_decode(q, k, v, causal, sm_scale, want_lse):
+    fast = _lib.native() if timing_events is None else None
+    if fast is not None:
+        done = fast.contiguous(q, k, v, causal, sm_scale, want_lse)
+        if done is not None:
+            return done
     _require(q.dim() == 4 and k.dim() == 4 and v.dim() == 4, "q, k, v must be [B, H, T, D]")
     batch, h_q, m, d = q.shape
     _require(k.shape[-1] == d and v.shape[-1] == d, "feature size of q, k, v should be equal")

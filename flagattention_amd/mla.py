@@ -133,6 +133,12 @@ def get_mla_metadata(
     metadata drives a sparse decode into skipped segments, sparse metadata a dense one
     into attending only the first ``ceil(topk / 64)`` pages).
     """
+    fast = _lib.native()
+    if fast is not None:
+        done = fast.mla_metadata(cache_seqlens, num_q_tokens_per_head_k, num_heads_k, num_heads_q,
+                                 topk, num_sm_parts)
+        if done is not None:
+            return done
     _require(isinstance(cache_seqlens, torch.Tensor), "cache_seqlens must be a tensor")
     _require(cache_seqlens.dtype == torch.int32, "cache_seqlens must be int32")
     _require(cache_seqlens.dim() == 1, "cache_seqlens must be 1-D [batch]")
@@ -362,6 +368,13 @@ def flash_mla_with_kvcache(
     Returns ``out`` bf16 [B, s_q, h_q, 512] and ``lse`` fp32 [B, h_q, s_q]; rows with no
     visible key get out = 0, lse = -inf.
     """
+    fast = _lib.native()
+    if fast is not None:
+        done = fast.mla_decode(q, k_cache, block_table, cache_seqlens, head_dim_v,
+                               tile_scheduler_metadata, num_splits, softmax_scale, causal,
+                               is_fp8_kvcache, indices)
+        if done is not None:
+            return done
     batch, s_q, h_q = _check_decode_args(q, k_cache, block_table, cache_seqlens, head_dim_v,
                                          tile_scheduler_metadata, num_splits, causal,
                                          is_fp8_kvcache, indices)
@@ -471,6 +484,9 @@ def concat_and_cache_mla(
     ``x / scale`` rounded to nearest even -- the layout ``flash_mla_with_kvcache(...,
     is_fp8_kvcache=True)`` reads.  Runs on the current stream; no host synchronisation.
     """
+    fast = _lib.native()
+    if fast is not None and fast.cache_write(kv_c, k_pe, kv_cache, slot_mapping, is_fp8_kvcache):
+        return
     _require(kv_c.dim() == 2 and kv_c.shape[1] == D_V and kv_c.dtype == torch.bfloat16,
              "kv_c must be bf16 [num_tokens, 512]")
     t = kv_c.shape[0]
@@ -536,6 +552,11 @@ def topk_indices(
     (-NaN < -inf < -0 < +0 < +inf < +NaN), ties by lower position, so the result is
     deterministic.  Runs on the current stream; no host synchronisation.
     """
+    fast = _lib.native() if out is None else None
+    if fast is not None:
+        done = fast.topk_indices(scores, cache_seqlens, topk, causal)
+        if done is not None:
+            return done
     _require(isinstance(scores, torch.Tensor) and scores.dim() == 3
              and scores.dtype == torch.float32, "scores must be float32 [batch, s_q, len]")
     batch, s_q, length = scores.shape
