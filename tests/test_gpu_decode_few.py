@@ -80,3 +80,19 @@ def test_dense_strided_q_and_cache():
                                                 ns, SCALE, True)
     torch.cuda.synchronize()
     assert_close(out.cpu(), lse.cpu(), *ref)
+
+
+@pytest.mark.parametrize("B,h_q,lens,parts", [
+    (1, 16, [9000], None),               # one sequence over every part: 8 waves per row
+    (3, 40, [2500, 0, 700], None),       # 85 parts per sequence at most, an empty sequence
+    (12, 5, [900] * 11 + [1], 240),      # 20 per sequence: 4 waves; one of a single split
+    (2, 130, [3000, 64], 18),            # 9 per sequence, more rows than a work-group
+    (2, 16, [3000, 64], 16),             # 8 per sequence: one wave per row
+])
+def test_dense_combine_many_splits(B, h_q, lens, parts):
+    """Split counts on both sides of the combine's choices of waves per row."""
+    need_gpu()
+    q, kc, bt, ld = orc.make_dense_inputs(B, h_q, 1, lens, seed=B + h_q, scale=1.0,
+                                          extra_blocks=1)
+    out, lse, _, _ = run_dense(q, kc, bt, ld, SCALE, False, parts)
+    assert_close(out, lse, *dense_refs(q, kc, bt, ld, SCALE, False))
