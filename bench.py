@@ -780,7 +780,10 @@ def run_mla(args) -> dict | None:
     if not args.no_cpu_baseline:
         cpu = cpu_baseline(spec, q, pools[0], tables[0], lens, indices)
 
-    step_kernels = ["mla_metadata_kernel"] + (["mla_sparse_rows_kernel"] if spec["topk"] else [])
+    # (a top-k list of up to FOLD_TOPK slots is translated to rows inside the decode)
+    from flagattention_amd.mla import FOLD_TOPK
+    step_kernels = ["mla_metadata_kernel"] + (
+        ["mla_sparse_rows_kernel"] if (spec["topk"] or 0) > FOLD_TOPK else [])
     step_kernels += ["mla_decode_kernel", "mla_combine_kernel"]
     rec = {
         "metric": METRIC,

@@ -84,9 +84,13 @@ struct __attribute__((aligned(16))) Smem {
   unsigned char p[kRows * 64];
   // Q^T operands that do not fit in VGPRs: [wave][operand][lane]
   bf16x8 qx[4][kQLds][64];
-  // sparse: each wave's ring of tile row lists, tile u in slot u % 3 (lanes
-  // 32..63 repeat rows 0..31)
-  int32_t rows[4][3][64];
+  // sparse: the segment's row ids, translated in the prologue (kFold); or each
+  // wave's ring of tile row lists, tile u in slot u % 3 (lanes 32..63 repeat
+  // rows 0..31)
+  union {
+    int32_t list[kFoldTopk];
+    int32_t rows[4][3][64];
+  };
 };
 
 // Source of masked gather rows: every lane issues its copy (so each wave has
@@ -164,7 +168,7 @@ __device__ inline void copy_block_buf(__amdgpu_buffer_rsrc_t rs, unsigned char* 
                                            voff, 0, 128 * G, kNonTemporal);
 }
 
-template <int kMode>
+template <int kMode, bool kFold>
 __global__ __launch_bounds__(kThreads, 1) void mla_decode_kernel(const fa_mla_decode_args a,
                                                                  int num_m_blocks) {
   // ring of three bf16 tiles (blocked layout); tile u lives in buffer u % 3
@@ -492,6 +496,7 @@ __global__ __launch_bounds__(kThreads, 1) void mla_decode_kernel(const fa_mla_de
       int32_t m, g;
     };
     auto request_rows = [&](int u) {
+      if constexpr (kFold) return;
       const int uu = u < ntiles ? u : ntiles - 1;
       const int ln = fresh_lane();  // rebuilt here: kept, the lane term is spilled
       lds_dma4(srows + tok_lo + kTileRows * uu + (ln & 31),
@@ -499,6 +504,11 @@ __global__ __launch_bounds__(kThreads, 1) void mla_decode_kernel(const fa_mla_de
     };
     auto read_rows = [&](int u) -> RowPair {  // after a wait that covers request_rows(u)
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kFold) {
+        const int32_t* const l = sm.list + kTileRows * (u < ntiles ? u : ntiles - 1);
+        const int ln = fresh_lane();  // offsets kept from the kernel start are spilled
+        return RowPair{l[ln & 31], l[8 * wave + (ln >> 3)]};
+      }
       const int32_t* ring = sm.rows[wave][u % 3];
       return RowPair{ring[lane & 31], ring[8 * wave + lrow]};
     };
@@ -577,8 +587,16 @@ __global__ __launch_bounds__(kThreads, 1) void mla_decode_kernel(const fa_mla_de
         // landed (it does not see the row and tile loads, so a wait for part
         // of Q would come out as a full wait inside the loop).  (Requesting Q
         // behind the first copies instead measured 3% slower.)
-        if (with_q) load_q();  // uniform
+        // kFold: the segment's slots are translated here instead (once: the list
+        // stays for the second pass), Q requested behind their page lookups.
+        if constexpr (kFold) {
+          if (with_q)  // uniform
+            fold_rows(a, b, s_fix, seqlen, tok_lo, ntiles * kTileRows, wave, sm.list, load_q);
+        } else {
+          if (with_q) load_q();  // uniform
+        }
         wait_vmem<0>();
+        if constexpr (kFold) barrier();
         const RowPair r0 = row_valid(0, read_rows(0)), r1 = row_valid(1, read_rows(1));
         vq[0] = row_mask(r0);
         vq[1] = row_mask(r1);
@@ -640,7 +658,7 @@ __global__ __launch_bounds__(kThreads, 1) void mla_decode_kernel(const fa_mla_de
         if constexpr (kMode != kSparseFp8 && !kPrevIssued) {
           wait_vmem<0>();  // nothing of tile t+1 was requested after tile t
         } else if constexpr (kMode == kSparseBf16) {
-          wait_vmem<kCopiesPerWave + 1>();  // also the rows of tile t+2 (one load)
+          wait_vmem<kCopiesPerWave + !kFold>();  // also the rows of tile t+2 (one load)
         } else if constexpr (kMode == kDense) {
           wait_vmem<kCopiesPerWave>();
         }
@@ -851,7 +869,7 @@ __global__ __launch_bounds__(kThreads, 1) void mla_decode_kernel(const fa_mla_de
           Fp8Codes dq;
           if constexpr (kMode == kSparseFp8) {
             if constexpr (kIssue) {
-              wait_vmem<kFp8Copies + 1>();  // tile t+2's copies and rows may be in flight
+              wait_vmem<kFp8Copies + !kFold>();  // tile t+2's copies and rows may be in flight
             } else {
               wait_vmem<0>();
             }
@@ -1110,16 +1128,16 @@ int check_common(const fa_mla_decode_args* a) {
   return FA_OK;
 }
 
-template <int kMode>
+template <int kMode, bool kFold>
 int launch_decode(const fa_mla_decode_args* a, hipStream_t stream) {
   // dense: flattened (s, h) rows; sparse: one query token per work-group
   const int num_m_blocks = kMode == kDense ? cdiv(a->s_q * a->h_q, kRows)
                                            : a->s_q * cdiv(a->h_q, kRows);
   // rows that share one KV stream: few of them leave the 128-row kernel mostly idle
   if ((kMode == kDense ? static_cast<long long>(a->s_q) * a->h_q : a->h_q) <= kFewRowsMax)
-    return launch_decode_few(a, kMode, stream);
+    return launch_decode_few(a, kMode, kFold, stream);
   const int grid = a->num_parts * num_m_blocks;
-  hipLaunchKernelGGL(mla_decode_kernel<kMode>, dim3(grid), dim3(kThreads), 0, stream, *a,
+  hipLaunchKernelGGL((mla_decode_kernel<kMode, kFold>), dim3(grid), dim3(kThreads), 0, stream, *a,
                      num_m_blocks);
   FA_CHECK_HIP(hipGetLastError());
   return FA_OK;
@@ -1135,7 +1153,7 @@ extern "C" int fa_mla_decode_dense(const fa_mla_decode_args* a, void* stream) {
                static_cast<long long>(a->kv_row_stride));
   FA_CHECK_ARG(a->max_blocks_per_seq >= 1, "block_table has %d columns (needs >= 1)",
                a->max_blocks_per_seq);
-  return fa::launch_decode<fa::kDense>(a, static_cast<hipStream_t>(stream));
+  return fa::launch_decode<fa::kDense, false>(a, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int fa_mla_sparse_rows(const fa_mla_decode_args* a, void* stream) {
@@ -1163,15 +1181,21 @@ extern "C" int fa_mla_sparse_rows(const fa_mla_decode_args* a, void* stream) {
 extern "C" int fa_mla_decode_sparse(const fa_mla_decode_args* a, int32_t fp8, void* stream) {
   int rc = fa::check_common(a);
   if (rc != FA_OK) return rc;
-  FA_CHECK_ARG(a->sparse_rows != nullptr, "sparse decode needs sparse_rows (fa_mla_sparse_rows)");
+  const bool fold = a->sparse_rows == nullptr;
+  FA_CHECK_ARG(!fold || (a->indices && a->topk <= FA_MLA_FOLD_TOPK && a->num_kv_blocks >= 1),
+               "sparse decode needs sparse_rows (fa_mla_sparse_rows), or indices with topk <= %d",
+               FA_MLA_FOLD_TOPK);
+  const hipStream_t st = static_cast<hipStream_t>(stream);
   FA_CHECK_ARG(a->topk >= 1, "topk %d < 1", a->topk);
   FA_CHECK_ARG(!a->causal, "causal masking does not apply to sparse decode");
   if (fp8) {
     FA_CHECK_ARG(a->kv_row_stride >= fa::kFp8RowBytes, "fp8 kv_row_stride %lld < 656",
                  static_cast<long long>(a->kv_row_stride));
-    return fa::launch_decode<fa::kSparseFp8>(a, static_cast<hipStream_t>(stream));
+    return fold ? fa::launch_decode<fa::kSparseFp8, true>(a, st)
+                : fa::launch_decode<fa::kSparseFp8, false>(a, st);
   }
   FA_CHECK_ARG(a->kv_row_stride >= 2 * fa::kDqk, "kv_row_stride %lld < 1152",
                static_cast<long long>(a->kv_row_stride));
-  return fa::launch_decode<fa::kSparseBf16>(a, static_cast<hipStream_t>(stream));
+  return fold ? fa::launch_decode<fa::kSparseBf16, true>(a, st)
+              : fa::launch_decode<fa::kSparseBf16, false>(a, st);
 }

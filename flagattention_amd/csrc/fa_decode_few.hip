@@ -58,13 +58,15 @@ __device__ inline void buf_lds16_nt(uintx4 rsrc, unsigned int voff, unsigned int
                : "memory", "m0");
 }
 
-template <int kMode, int NR>
+template <int kMode, int NR, bool kFold>
 __global__ __launch_bounds__(kThreads, 2) void mla_decode_few_kernel(const fa_mla_decode_args a,
                                                                      int num_m_blocks) {
   __shared__ __attribute__((aligned(16))) unsigned char tiles[kFewRing * kTileBytes];
   // S pieces: [tile parity][k-step half or row tile][16-key half][lane]
   __shared__ floatx4 sx[2][2][2][64];
-  __shared__ int32_t row_ring[kMode == kDense ? 1 : 4][kFewRing][64];  // sparse: per wave
+  // sparse: the segment's translated row ids (kFold), or each wave's ring of tile row lists
+  __shared__ int32_t row_list[kFold ? kFoldTopk : 1];
+  __shared__ int32_t row_ring[kMode == kDense || kFold ? 1 : 4][kFold ? 1 : kFewRing][64];
 
   // XCD-aware work-group -> (part, query token), as in the 128-row kernel
   const int wg = blockIdx.x;
@@ -159,6 +161,7 @@ __global__ __launch_bounds__(kThreads, 2) void mla_decode_few_kernel(const fa_ml
     };
     int page_next = -1;
     auto request_rows = [&](int u) {  // sparse: tile u's row list into this wave's ring
+      if constexpr (kFold) return;
       lds_dma4(srows + tok_lo + kTileRows * u + (lane & 31),
                (FA_LDS void*)(&row_ring[wave][u & 3][0]));
     };
@@ -184,7 +187,7 @@ __global__ __launch_bounds__(kThreads, 2) void mla_decode_few_kernel(const fa_ml
           buf_lds16_nt(rs, page_voff, 128 * c, (FA_LDS void*)(dst + c * kBlockBytes));
         return nrows >= kTileRows ? ~0u : ((1u << nrows) - 1u);
       } else {
-        const int32_t* const ring = row_ring[wave][u & 3];
+        const int32_t* const ring = kFold ? row_list + kTileRows * u : row_ring[wave][u & 3];
         const int32_t rm = ring[lane & 31], r = ring[8 * wave + lrow];
         const unsigned int rr = static_cast<unsigned int>(r < 0 ? 0 : r);
         const unsigned char* src =
@@ -214,7 +217,7 @@ __global__ __launch_bounds__(kThreads, 2) void mla_decode_few_kernel(const fa_ml
     // read zeros.
     unsigned char* const qbuf = tiles + (kFewRing - 1) * kTileBytes;
     static_assert(NR * kQkSteps * kBlockBytes <= kTileBytes, "Q fits one tile buffer");
-    {
+    auto load_q = [&] {
       constexpr int kOps = NR * kQkSteps, kPerWave = (kOps + 3) / 4;
 #pragma unroll
       for (int i = 0; i < kPerWave; ++i) {
@@ -230,10 +233,17 @@ __global__ __launch_bounds__(kThreads, 2) void mla_decode_few_kernel(const fa_ml
                             : g_few_zero;
         lds_dma16(src, (FA_LDS void*)(qbuf + j * kBlockBytes));
       }
-    }
+    };
+    if constexpr (!kFold) load_q();
     unsigned int vm[4] = {0u, 0u, 0u, 0u};  // key masks of tiles t .. t+3
     if constexpr (kMode == kDense) {
       page_next = load_page(0);
+    } else if constexpr (kFold) {
+      fold_rows(a, b, mb, seqlen, tok_lo, ntiles * kTileRows, wave, row_list, load_q);
+      wait_vmem<0>();
+      asm volatile("" ::: "memory");
+      barrier();
+      asm volatile("" ::: "memory");
     } else {
       for (int u = 0; u < min(ntiles, 4); ++u) request_rows(u);
       wait_vmem<0>();
@@ -459,28 +469,28 @@ __global__ __launch_bounds__(kThreads, 2) void mla_decode_few_kernel(const fa_ml
   }
 }
 
-template <int kMode>
+template <int kMode, bool kFold>
 void launch_few(const fa_mla_decode_args* a, hipStream_t stream) {
   const int rows = kMode == kDense ? a->s_q * a->h_q : a->h_q;
   const int num_m_blocks = kMode == kDense ? 1 : a->s_q;
   const dim3 grid(static_cast<unsigned>(a->num_parts * num_m_blocks));
   if (rows <= 16)
-    hipLaunchKernelGGL((mla_decode_few_kernel<kMode, 1>), grid, dim3(kThreads), 0, stream, *a,
+    hipLaunchKernelGGL((mla_decode_few_kernel<kMode, 1, kFold>), grid, dim3(kThreads), 0, stream, *a,
                        num_m_blocks);
   else
-    hipLaunchKernelGGL((mla_decode_few_kernel<kMode, 2>), grid, dim3(kThreads), 0, stream, *a,
+    hipLaunchKernelGGL((mla_decode_few_kernel<kMode, 2, kFold>), grid, dim3(kThreads), 0, stream, *a,
                        num_m_blocks);
 }
 
 }  // namespace
 
-int launch_decode_few(const fa_mla_decode_args* a, int mode, hipStream_t stream) {
+int launch_decode_few(const fa_mla_decode_args* a, int mode, bool fold, hipStream_t stream) {
   if (mode == kDense)
-    launch_few<kDense>(a, stream);
+    launch_few<kDense, false>(a, stream);
   else if (mode == kSparseBf16)
-    launch_few<kSparseBf16>(a, stream);
+    fold ? launch_few<kSparseBf16, true>(a, stream) : launch_few<kSparseBf16, false>(a, stream);
   else
-    launch_few<kSparseFp8>(a, stream);
+    fold ? launch_few<kSparseFp8, true>(a, stream) : launch_few<kSparseFp8, false>(a, stream);
   FA_CHECK_HIP(hipGetLastError());
   return FA_OK;
 }

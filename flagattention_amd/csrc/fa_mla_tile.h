@@ -108,8 +108,48 @@ __device__ inline void dequant_fp8_rowgroup(unsigned char* buf, int wave) {
   });
 }
 
+// Sparse index translation inside the decode (topk <= FA_MLA_FOLD_TOPK): at the start of a
+// segment the work-group turns its index slots into physical cache rows, -1 where masked, in
+// an LDS list (the arithmetic of mla_sparse_rows_kernel).  512 slots at a time, two per
+// thread.  Against a launch of its own in front of the decode (3.8 us and its gap): sparse
+// top-2,048 steps of 64 sequences, bf16, 67.4 -> 64.7 us, of 128, fp8, 106.4 -> 104.3 (the
+// decode itself 1 us longer).  The limit is the LDS that the 32-row kernel's tiles leave
+// (8 KB).  between() is called once, after the first page lookups have been issued and before
+// they are waited for, so that the caller's own loads overlap them.
+constexpr int kFoldTopk = FA_MLA_FOLD_TOPK;
+template <typename F>
+__device__ inline void fold_rows(const fa_mla_decode_args& a, int b, int s, int seqlen, int tok_lo,
+                                 int nslots, int wave, int32_t* list, F&& between) {
+  const int32_t* const row = a.indices + b * a.idx_stride_b + s * a.idx_stride_s;
+  const int32_t* const bt = a.block_table + static_cast<long long>(b) * a.bt_stride_b;
+  auto part = [&](int k0, auto&& mid) {
+    const int tid = 64 * wave + fresh_lane();  // rebuilt: kept, it is spilled
+    int32_t idx[2], page[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int k = k0 + kThreads * i + tid;
+      idx[i] = k < nslots && tok_lo + k < a.topk ? row[tok_lo + k] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const bool ok = idx[i] >= 0 && idx[i] < seqlen && (idx[i] >> 6) < a.max_blocks_per_seq;
+      page[i] = ok ? bt[idx[i] >> 6] : -1;
+    }
+    mid();
+    const int tid2 = 64 * wave + fresh_lane();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int k = k0 + kThreads * i + tid2;
+      if (k < nslots)
+        list[k] = page[i] >= 0 && page[i] < a.num_kv_blocks ? page[i] * kPage + (idx[i] & 63) : -1;
+    }
+  };
+  part(0, between);
+  for (int k0 = 2 * kThreads; k0 < nslots; k0 += 2 * kThreads) part(k0, [] {});
+}
+
 // Decode of up to kFewRowsMax query rows per KV stream (fa_decode_few.hip).
 constexpr int kFewRowsMax = 32;
-int launch_decode_few(const fa_mla_decode_args* a, int mode, hipStream_t stream);
+int launch_decode_few(const fa_mla_decode_args* a, int mode, bool fold, hipStream_t stream);
 
 }  // namespace fa

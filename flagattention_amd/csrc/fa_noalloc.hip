@@ -81,10 +81,12 @@ extern "C" int fa_mla_decode_noalloc(const fa_mla_decode_args* a, int32_t mode, 
   w.o_accum = base;
   w.lse_accum = reinterpret_cast<float*>(base + fa::align256(segs * rows * fa::kDv * 2));
   if (mode != 0) {
-    w.sparse_rows = reinterpret_cast<int32_t*>(base + fa::align256(segs * rows * fa::kDv * 2) +
-                                               fa::align256(segs * rows * 4));
-    rc = fa_mla_sparse_rows(&w, stream);
-    if (rc != FA_OK) return rc;
+    if (w.topk > FA_MLA_FOLD_TOPK) {  // up to it the decode translates its slots itself
+      w.sparse_rows = reinterpret_cast<int32_t*>(base + fa::align256(segs * rows * fa::kDv * 2) +
+                                                 fa::align256(segs * rows * 4));
+      rc = fa_mla_sparse_rows(&w, stream);
+      if (rc != FA_OK) return rc;
+    }
     rc = fa_mla_decode_sparse(&w, mode == 2 ? 1 : 0, stream);
   } else {
     rc = fa_mla_decode_dense(&w, stream);

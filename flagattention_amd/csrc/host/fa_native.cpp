@@ -254,7 +254,8 @@ PyObject* mla_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // one workspace: partial outputs (bf16), their lse (fp32), gather rows (int32)
     const int64_t o_bytes = (batch + parts) * rows * FA_MLA_D_V * 2;
     const int64_t lse_bytes = cdiv((batch + parts) * rows * 4, 256) * 256;
-    const int64_t row_bytes = sparse ? batch * s_q * cdiv(topk, kPage) * kPage * 4 : 0;
+    // row ids only where the decode does not translate its slots itself
+    const int64_t row_bytes = topk > FA_MLA_FOLD_TOPK ? batch * s_q * cdiv(topk, kPage) * kPage * 4 : 0;
     const at::Tensor ws = make({o_bytes + lse_bytes + row_bytes}, at::kByte, device);
     uint8_t* const w = ws.data_ptr<uint8_t>();
     fa_mla_decode_args a = {};
@@ -288,8 +289,10 @@ PyObject* mla_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       a.idx_stride_b = idx->stride(0);
       a.idx_stride_s = idx->stride(1);
       a.topk = static_cast<int32_t>(topk);
-      a.sparse_rows = reinterpret_cast<int32_t*>(w + o_bytes + lse_bytes);
-      check(fa_mla_sparse_rows(&a, stream));
+      if (topk > FA_MLA_FOLD_TOPK) {
+        a.sparse_rows = reinterpret_cast<int32_t*>(w + o_bytes + lse_bytes);
+        check(fa_mla_sparse_rows(&a, stream));
+      }
       check(fa_mla_decode_sparse(&a, fp8, stream));
     } else {
       check(fa_mla_decode_dense(&a, stream));

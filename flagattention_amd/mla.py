@@ -41,6 +41,9 @@ MD_STRIDE = 8
 FP8_ROW_BYTES = 656
 MAX_BATCH = 4096
 MAX_PARTS = 1024
+# Sparse decode of up to this topk translates its index slots to cache rows itself; longer
+# lists are translated by a launch of their own into a workspace.
+FOLD_TOPK = 2048
 # Scheduler cost, in 64-token blocks, charged once per sequence on the cost line
 # (a sequence start inside a part adds a segment there: Q load, partial write-out and
 # its share of the combine).
@@ -275,7 +278,8 @@ class DecodeWorkspace:
     benchmark) can keep one and call :meth:`run` every step, so no allocation happens
     per step.  Buffers: ``out`` bf16 [B, s_q, h_q, 512], ``lse`` fp32 [B, h_q, s_q],
     ``o_accum`` bf16 [B + parts, s_q * h_q, 512], ``lse_accum`` fp32 [B + parts, s_q * h_q]
-    and, for sparse decode, the gather rows int32 [B, s_q, ceil(topk / 64) * 64].
+    and, for sparse decode with topk > FOLD_TOPK, the gather rows int32
+    [B, s_q, ceil(topk / 64) * 64] (``rows``, else None).
     """
 
     def __init__(self, batch: int, s_q: int, h_q: int, num_parts: int,
@@ -290,7 +294,7 @@ class DecodeWorkspace:
         self.lse_accum = torch.empty((batch + num_parts, rows), dtype=torch.float32,
                                      device=device)
         self.rows = None
-        if topk is not None:
+        if topk is not None and topk > FOLD_TOPK:
             topk_pad = -(-topk // PAGE_SIZE) * PAGE_SIZE
             self.rows = torch.empty((batch, s_q, topk_pad), dtype=torch.int32, device=device)
 
@@ -326,8 +330,9 @@ class DecodeWorkspace:
             stream = _stream(device)
             if indices is not None:
                 _set_indices(args, indices)
-                args.sparse_rows = self.rows.data_ptr()
-                _lib.check(lib.fa_mla_sparse_rows(ctypes.byref(args), stream))
+                if self.rows is not None:
+                    args.sparse_rows = self.rows.data_ptr()
+                    _lib.check(lib.fa_mla_sparse_rows(ctypes.byref(args), stream))
             if decode_events is not None:
                 decode_events[0].record()
             if indices is None:

@@ -39,6 +39,7 @@ extern "C" {
 #define FA_MLA_MD_STRIDE 8   /* int32 words per tile-scheduler entry     */
 #define FA_MLA_FP8_ROW_BYTES 656 /* 512 e4m3 + 4 fp32 scales + 64 bf16   */
 #define FA_MLA_MAX_BATCH 4096
+#define FA_MLA_FOLD_TOPK 2048 /* sparse decode translates up to this topk itself */
 #define FA_MLA_MAX_PARTS 1024
 /* Workspace of fa_mla_decode_noalloc: one file-scope device array of this
  * many bytes per device the library runs on, held until the process ends. */
@@ -154,7 +155,9 @@ int fa_mla_sparse_rows(const fa_mla_decode_args* args, void* stream);
 
 /*
  * Sparse top-k decode: each query token attends only to the cache rows in
- * args->sparse_rows (from fa_mla_sparse_rows); -1 rows are masked.
+ * args->sparse_rows (from fa_mla_sparse_rows); -1 rows are masked.  With
+ * sparse_rows NULL and topk <= FA_MLA_FOLD_TOPK the decode translates
+ * args->indices itself (no fa_mla_sparse_rows call needed).
  * fp8 != 0 selects the 656-byte fp8-e4m3 row layout (512 codes, 4 fp32
  * per-128-dim scales, 64 bf16 rope dims; dequantised on chip), else the
  * 1152-byte bf16 row.  No reference counterpart (the reference has no sparse

@@ -96,3 +96,22 @@ def test_dense_combine_many_splits(B, h_q, lens, parts):
                                           extra_blocks=1)
     out, lse, _, _ = run_dense(q, kc, bt, ld, SCALE, False, parts)
     assert_close(out, lse, *dense_refs(q, kc, bt, ld, SCALE, False))
+
+
+@pytest.mark.parametrize("h_q", [16, 32, 48])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("topk,parts", [(2047, 1), (2048, 1), (2048, 3), (2049, 1), (513, 1)])
+def test_sparse_translation_limit(h_q, fp8, topk, parts):
+    """Index lists on both sides of the in-kernel translation's limit and of its 512-slot
+    rounds, with page ids outside the cache and ids past the length among them."""
+    need_gpu()
+    lens = [2600, 700]
+    q, kc, bt, ld = orc.make_dense_inputs(2, h_q, 1, lens, seed=topk, scale=1.0, extra_blocks=1)
+    if fp8:
+        kc = orc.make_fp8_cache(kc.shape[0], seed=topk + 7, lat_scale=1.0)
+    idx = torch.randint(-3, 2700, (2, 1, topk),
+                        generator=torch.Generator().manual_seed(topk)).to(torch.int32)
+    bt = bt.clone()
+    bt[0, 3], bt[1, 0] = kc.shape[0], -1
+    out, lse = run_sparse(q, kc, bt, ld, idx, SCALE, fp8, parts)
+    assert_close(out, lse, *sparse_refs(q, kc, bt, ld, idx, SCALE, fp8))
