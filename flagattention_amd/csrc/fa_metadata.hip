@@ -33,32 +33,38 @@ constexpr int kMaxB = FA_MLA_MAX_BATCH;
 constexpr int kMaxP = FA_MLA_MAX_PARTS;
 static_assert(kMaxP <= kMetaThreadsMax && kMaxB <= 4 * kMetaThreadsMax, "one block covers a call");
 
-// Inclusive prefix sums over the work-group of a 64-bit and a 32-bit value
+__device__ inline long long wave_scan(long long x) { return wave_incl_scan64(x); }
+__device__ inline int wave_scan(int x) { return wave_incl_scan(x); }
+
+// Inclusive prefix sums over the work-group of a value of type I and a 32-bit value
 // (one pair per thread): DPP scans inside each wave (no LDS round trips), then
 // the totals of the waves before this one read back from LDS (broadcast reads;
-// two barriers; `sh64` / `sh32` are free again on return).
-template <int kWaves>
-__device__ void block_incl_scan2(long long& v, int& k, long long* sh64, int* sh32) {
+// two barriers; `shv` / `sh32` are free again on return).  Returns the total of k.
+template <typename I, int kWaves>
+__device__ int block_incl_scan2(I& v, int& k, I* shv, int* sh32) {
   const int lane = threadIdx.x & 63, w = wave_id();
-  v = wave_incl_scan64(v);
+  v = wave_scan(v);
   k = wave_incl_scan(k);
   if (lane == 63) {
-    sh64[w] = v;
+    shv[w] = v;
     sh32[w] = k;
   }
   __syncthreads();
-  long long bv = 0;
-  int bk = 0;
+  I bv = 0;
+  int bk = 0, total = 0;
 #pragma unroll
-  for (int i = 0; i < kWaves - 1; ++i) {
+  for (int i = 0; i < kWaves; ++i) {
+    const int ki = sh32[i];
     if (i < w) {  // uniform
-      bv += sh64[i];
-      bk += sh32[i];
+      bv += shv[i];
+      bk += ki;
     }
+    total += ki;
   }
   __syncthreads();
   v += bv;
   k += bk;
+  return total;
 }
 
 // block_incl_scan2 of a 32-bit value alone.
@@ -81,7 +87,8 @@ __device__ void block_incl_scan(int& k, int* sh32) {
 // the answer lies in [lo, hi) with a[lo] <= x; each round probes lo + k * step for
 // k = 1..7 (seven independent LDS reads, one latency per round instead of one per
 // halving), and the probes that pass form a prefix.  n <= 64 takes two rounds.
-__device__ int last_le(const long long* a, int n, long long x) {
+template <typename I>
+__device__ int last_le(const I* a, int n, I x) {
   int lo = 0, hi = n;
   while (hi - lo > 1) {
     const int step = (hi - lo + 7) >> 3;
@@ -89,7 +96,7 @@ __device__ int last_le(const long long* a, int n, long long x) {
 #pragma unroll
     for (int k = 1; k < 8; ++k) {
       const int p = lo + k * step;
-      const long long v = a[p < hi ? p : hi - 1];
+      const I v = a[p < hi ? p : hi - 1];
       cnt += (p < hi && v <= x) ? 1 : 0;
     }
     lo += cnt * step;
@@ -110,11 +117,170 @@ __device__ inline long long floor_div(long long a, long long b, double rb) {
   return q;
 }
 
-__device__ inline long long seq_blocks(const int32_t* lens, int b, int topk) {
-  if (topk > 0) return (topk + kPage - 1) / kPage;
-  const int len = lens[b];
-  return len > 0 ? (len + kPage - 1) / kPage : 0;
+// Cuts of the cost line, x_p = ceil(p W / P), and the last part whose cut is <= c.
+// 64-bit: both divisions by double estimates.
+template <typename I>
+struct Cuts;
+template <>
+struct Cuts<long long> {
+  long long W;
+  int P;
+  double rP, rW;
+  __device__ Cuts(long long w, int p)
+      : W(w), P(p), rP(1.0 / static_cast<double>(p)), rW(1.0 / static_cast<double>(w > 0 ? w : 1)) {}
+  __device__ long long at(int p) const {
+    // x_P = W exactly: no division for the last cut (with P = threads it is the one
+    // part a thread would otherwise take second)
+    return p == P ? W : floor_div(static_cast<long long>(p) * W + P - 1, P, rP);
+  }
+  __device__ int last_at_or_before(long long c) const {
+    return static_cast<int>(floor_div(c * P, W, rW));
+  }
+};
+// 32-bit (W < 2^30, P <= 2^10): W = wq P + wr gives x_p = p wq + ceil(p wr / P), whose
+// quotient stays below 2^21, exact from a float estimate and one correction; the part of a
+// position c comes from the float estimate c P / W (below 2^10, so within 1) and the cuts
+// beside it.
+template <>
+struct Cuts<int> {
+  int W, P, wq, wr;
+  float rP, rW;
+  __device__ Cuts(int w, int p) : W(w), P(p), wq(w / p), wr(w - w / p * p) {
+    rP = 1.f / static_cast<float>(p);
+    rW = static_cast<float>(p) / static_cast<float>(w > 0 ? w : 1);
+  }
+  __device__ int at(int p) const {
+    const int n = p * wr + P - 1;
+    int q = static_cast<int>(static_cast<float>(n) * rP);
+    if (q * P > n) --q;
+    if ((q + 1) * P <= n) ++q;
+    return p * wq + q;
+  }
+  __device__ int last_at_or_before(int c) const {
+    int q = min(static_cast<int>(static_cast<float>(c) * rW), P);
+    if (at(q) > c) --q;
+    if (q < P && at(q + 1) <= c) ++q;
+    return q;
+  }
+};
+
+// The partition, in block-count type I (see the file comment): C, G, gs are prefix arrays in
+// LDS, ginc / kinc this thread's inclusive sums of blocks and of non-empty sequences.
+template <typename I, int kMetaThreads>
+__device__ void partition(const int (&nbs)[4], int b0, int b1, I ginc, I gsum, int kinc, int ksum,
+                          int B, int P, int overhead, int32_t* __restrict__ md,
+                          int32_t* __restrict__ num_splits, I* C, I* G, I* gs, int* pf, int* pl,
+                          int* owner, int* E, int* sh32) {
+  constexpr int kMetaWaves = kMetaThreads / 64;
+  const int t = threadIdx.x;
+  // 1. G and C[b] = G[b] + overhead * (non-empty sequences before b)
+  {
+    I gg = ginc - gsum;
+    int kk = kinc - ksum;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (b0 + i < b1) {
+        G[b0 + i] = gg;
+        C[b0 + i] = gg + static_cast<I>(overhead) * kk;
+        gg += nbs[i];
+        kk += nbs[i] > 0;
+      }
+    }
+    if (t == kMetaThreads - 1) {
+      G[B] = ginc;
+      C[B] = ginc + static_cast<I>(overhead) * kinc;
+    }
+  }
+  __syncthreads();
+  const I W = C[B];
+  const I NB = G[B];
+  const Cuts<I> cuts(W, P);
+
+  // 2. part starts x_p = ceil(p W / P) on the cost line -> global blocks; and
+  //    per sequence, the parts that hold its first and last block, in closed
+  //    form: gs_p <= G[b] exactly when x_p <= C[b] + overhead, and
+  //    gs_p < G[b+1] exactly when x_p < C[b+1], and x_p grows with p.
+  for (int p = t; p <= P; p += kMetaThreads) {
+    const I x = cuts.at(p);
+    I v;
+    int own;
+    if (x >= W) {
+      v = NB;
+      own = B;
+    } else {
+      own = last_le(C, B, x);
+      const I o = x - C[own] - overhead;
+      v = G[own] + (o > 0 ? o : 0);
+    }
+    gs[p] = v;
+    owner[p] = own;
+  }
+  for (int b = b0; b < b1; ++b) {
+    if (G[b + 1] > G[b]) {
+      pf[b] = cuts.last_at_or_before(C[b] + overhead);
+      pl[b] = cuts.last_at_or_before(C[b + 1] - 1);
+    }
+  }
+  __syncthreads();
+
+  // 3. E[p] = number of empty parts in [0, p).
+  {
+    const int cnt = (t < P && gs[t] == gs[t + 1]) ? 1 : 0;
+    int inc = cnt;
+    block_incl_scan<kMetaWaves>(inc, sh32);
+    if (t < P) E[t] = inc - cnt;
+    if (t == kMetaThreads - 1) E[P] = inc;
+  }
+  __syncthreads();
+
+  // 4. per-part descriptors: a non-empty part starts in the sequence whose
+  //    cost interval holds its x_p.
+  if (t < P) {
+    const I g0 = gs[t], g1 = gs[t + 1];
+    int4* m = reinterpret_cast<int4*>(md + static_cast<long long>(t) * kMdStride);
+    if (g0 == g1) {
+      m[0] = make_int4(0, 0, 0, 0);
+      m[1] = make_int4(0, 0, static_cast<int32_t>(g0), 0);
+    } else {
+      const int bb = owner[t];
+      const int eb = last_le(G, B, static_cast<I>(g1 - 1));
+      const int f = pf[bb];
+      m[0] = make_int4(bb, static_cast<int32_t>(g0 - G[bb]), eb, static_cast<int32_t>(g1 - G[eb]));
+      m[1] = make_int4((t - f) - (E[t] - E[f]), static_cast<int32_t>(g1 - g0),
+                       static_cast<int32_t>(g0), 0);
+    }
+  }
+
+  // 5. segments per sequence (non-empty parts from pf[b] to pl[b]) ->
+  //    exclusive prefix num_splits[B+1].
+  {
+    int segs[4];
+    int sum = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int b = b0 + i;
+      segs[i] = b < b1 && nbs[i] > 0 ? (pl[b] - pf[b] + 1) - (E[pl[b]] - E[pf[b]]) : 0;
+      sum += segs[i];
+    }
+    int inc = sum;
+    block_incl_scan<kMetaWaves>(inc, sh32);
+    int acc = inc - sum;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (b0 + i < b1) num_splits[b0 + i] = acc;
+      acc += segs[i];
+    }
+    if (t == kMetaThreads - 1) num_splits[B] = inc;
+  }
 }
+
+// The 32-bit partition runs when no sequence has 2^17 blocks (8.4M tokens) and the overhead
+// is at most 2^16, which keeps every sum below 2^30; the count of longer sequences rides in
+// the upper half of the non-empty count's scan.  Time per call in a replayed graph, 256 parts,
+// 64 bits / 32: 2 sequences 3.9 / 3.7 us, 64 4.3 / 4.0, 300 5.7 / 4.8 (what is left is the
+// chain of scans, searches and barriers).
+constexpr int kBigBlocks = 1 << 17;
+constexpr int kBigOverhead = 1 << 16;
 
 template <int kMetaThreads>
 __global__ __launch_bounds__(kMetaThreads) void mla_metadata_kernel(
@@ -133,117 +299,86 @@ __global__ __launch_bounds__(kMetaThreads) void mla_metadata_kernel(
 
   const int t = threadIdx.x;
   const int ipt = cdiv(B, kMetaThreads);  // sequences per thread (<= 4)
-  const double rP = 1.0 / static_cast<double>(P);
   const int b0 = min(B, t * ipt), b1 = min(B, b0 + ipt);
-
-  // 1. G and the count K of non-empty sequences, scanned together; then
-  //    C[b] = G[b] + overhead * K[b].
-  {
-    long long gsum = 0;
-    int ksum = 0;
-    for (int b = b0; b < b1; ++b) {
-      const long long nb = seq_blocks(lens, b, topk);
-      gsum += nb;
-      ksum += nb > 0;
-    }
-    long long ginc = gsum;
-    int kinc = ksum;
-    block_incl_scan2<kMetaWaves>(ginc, kinc, sh64, sh32);
-    long long gg = ginc - gsum;
-    long long kk = kinc - ksum;
-    for (int b = b0; b < b1; ++b) {
-      const long long nb = seq_blocks(lens, b, topk);
-      G[b] = gg;
-      C[b] = gg + overhead * kk;
-      gg += nb;
-      kk += nb > 0;
-    }
-    if (t == kMetaThreads - 1) {
-      G[B] = ginc;
-      C[B] = ginc + static_cast<long long>(overhead) * kinc;
-    }
+  int nbs[4];
+  int gsum = 0, ksum = 0;  // at most 4 * 2^25
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    // topk > 0: every sequence has topk slots
+    const int len = b0 + i < b1 ? (topk > 0 ? topk : lens[b0 + i]) : 0;
+    nbs[i] = len > 0 ? (len >> 6) + ((len & 63) != 0) : 0;
+    gsum += nbs[i];
+    ksum += (nbs[i] > 0) + ((nbs[i] >= kBigBlocks) << 16);
   }
-  __syncthreads();
-  const long long W = C[B];
-  const long long NB = G[B];
-  const double rW = 1.0 / static_cast<double>(W > 0 ? W : 1);
-
-  // 2. part starts x_p = ceil(p W / P) on the cost line -> global blocks; and
-  //    per sequence, the parts that hold its first and last block, in closed
-  //    form: gs_p <= G[b] exactly when x_p <= C[b] + overhead, and
-  //    gs_p < G[b+1] exactly when x_p < C[b+1], and x_p grows with p.
-  for (int p = t; p <= P; p += kMetaThreads) {
-    // x_P = W exactly: no division for the last cut (with P = threads it is the one
-    // part a thread would otherwise take second)
-    const long long x = p == P ? W : floor_div(static_cast<long long>(p) * W + P - 1, P, rP);
-    long long v;
-    int own;
-    if (x >= W) {
-      v = NB;
-      own = B;
-    } else {
-      own = last_le(C, B, x);
-      const long long o = x - C[own] - overhead;
-      v = G[own] + (o > 0 ? o : 0);
-    }
-    gs[p] = v;
-    owner[p] = own;
+  static_assert(kPage == 64, "blocks by shifts");
+  int ginc = gsum, kinc = ksum;
+  const int total = block_incl_scan2<int, kMetaWaves>(ginc, kinc, reinterpret_cast<int*>(sh64), sh32);
+  const bool big = (total >> 16) != 0 || overhead > kBigOverhead;  // uniform
+  if (!big) {
+    partition<int, kMetaThreads>(nbs, b0, b1, ginc, gsum, kinc, ksum, B, P, overhead, md,
+                                 num_splits, reinterpret_cast<int*>(C), reinterpret_cast<int*>(G),
+                                 reinterpret_cast<int*>(gs), pf, pl, owner, E, sh32);
+  } else {
+    long long ginc64 = gsum;
+    ksum &= 0xFFFF;
+    int kinc64 = ksum;
+    block_incl_scan2<long long, kMetaWaves>(ginc64, kinc64, sh64, sh32);
+    partition<long long, kMetaThreads>(nbs, b0, b1, ginc64, gsum, kinc64, ksum, B, P, overhead,
+                                       md, num_splits, C, G, gs, pf, pl, owner, E, sh32);
   }
-  for (int b = b0; b < b1; ++b) {
-    if (G[b + 1] > G[b]) {
-      pf[b] = static_cast<int>(floor_div((C[b] + overhead) * P, W, rW));
-      pl[b] = static_cast<int>(floor_div((C[b + 1] - 1) * P, W, rW));
-    }
-  }
-  __syncthreads();
+}
 
-  // 3. E[p] = number of empty parts in [0, p).
-  {
-    const int cnt = (t < P && gs[t] == gs[t + 1]) ? 1 : 0;
-    int inc = cnt;
-    block_incl_scan<kMetaWaves>(inc, sh32);
-    if (t < P) E[t] = inc - cnt;
-    if (t == kMetaThreads - 1) E[P] = inc;
-  }
-  __syncthreads();
-
-  // 4. per-part descriptors: a non-empty part starts in the sequence whose
-  //    cost interval holds its x_p.
+// Sparse: every sequence has T = ceil(topk / 64) blocks and costs nothing more, so W = NB =
+// B T and the values have closed forms: a part's cut is its first block, and the first and
+// last parts of a sequence come from the cuts.  Parts are empty only when P > W; then every
+// other part holds one block, and x_p parts before part p are not empty.  A sequence start
+// j T is also a part's start exactly when (P j mod B) T < P; the segments before sequence b
+// are the parts that start before b T plus one for every start in between that splits a
+// part -- the one scan here.  Time per call in a replayed graph, general
+// partition / this: 64 sequences of top-2,048, 256 parts 4.15 / 2.09 us.
+template <int kMetaThreads>
+__global__ __launch_bounds__(kMetaThreads) void mla_metadata_uniform_kernel(
+    int B, int T, int P, int32_t* __restrict__ md, int32_t* __restrict__ num_splits) {
+  constexpr int kMetaWaves = kMetaThreads / 64;
+  __shared__ int sh32[kMetaWaves];
+  const int t = threadIdx.x;
+  const int W = B * T;  // < 2^30 (host)
+  const Cuts<int> cuts(W, P);
+  auto used_before = [&](int p) { return P <= W ? p : cuts.at(p); };  // non-empty parts in [0, p)
   if (t < P) {
-    const long long g0 = gs[t], g1 = gs[t + 1];
+    const int g0 = cuts.at(t), g1 = cuts.at(t + 1);
     int4* m = reinterpret_cast<int4*>(md + static_cast<long long>(t) * kMdStride);
     if (g0 == g1) {
       m[0] = make_int4(0, 0, 0, 0);
-      m[1] = make_int4(0, 0, static_cast<int32_t>(g0), 0);
+      m[1] = make_int4(0, 0, g0, 0);
     } else {
-      const int bb = owner[t];
-      const int eb = last_le(G, B, g1 - 1);
-      const int f = pf[bb];
-      m[0] = make_int4(bb, static_cast<int32_t>(g0 - G[bb]), eb, static_cast<int32_t>(g1 - G[eb]));
-      m[1] = make_int4((t - f) - (E[t] - E[f]), static_cast<int32_t>(g1 - g0),
-                       static_cast<int32_t>(g0), 0);
+      const int bb = g0 / T, eb = (g1 - 1) / T;
+      const int f = cuts.last_at_or_before(bb * T);
+      m[0] = make_int4(bb, g0 - bb * T, eb, g1 - eb * T);
+      m[1] = make_int4(used_before(t) - used_before(f), g1 - g0, g0, 0);
     }
   }
-
-  // 5. segments per sequence (non-empty parts from pf[b] to pl[b]) ->
-  //    exclusive prefix num_splits[B+1].
-  {
-    int segs[4];
-    int sum = 0;
-    for (int b = b0; b < b1; ++b) {
-      const int n = G[b + 1] > G[b] ? (pl[b] - pf[b] + 1) - (E[pl[b]] - E[pf[b]]) : 0;
-      segs[b - b0] = n;
-      sum += n;
-    }
-    int inc = sum;
-    block_incl_scan<kMetaWaves>(inc, sh32);
-    int acc = inc - sum;
-    for (int b = b0; b < b1; ++b) {
-      num_splits[b] = acc;
-      acc += segs[b - b0];
-    }
-    if (t == kMetaThreads - 1) num_splits[B] = inc;
+  const int ipt = cdiv(B, kMetaThreads);  // <= 4
+  const int b0 = min(B, t * ipt), b1 = min(B, b0 + ipt);
+  int cut[4], sum = 0;  // starts that split a part
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int j = b0 + i;
+    cut[i] = j < b1 && j > 0 && static_cast<int>(static_cast<unsigned int>(P * j) % B) * T >= P;
+    sum += cut[i];
   }
+  int inc = sum;
+  block_incl_scan<kMetaWaves>(inc, sh32);
+  int acc = inc - sum;  // of the starts before b0
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int b = b0 + i;
+    if (b < b1)
+      num_splits[b] = b == 0 ? 0 : used_before(cuts.last_at_or_before(b * T - 1) + 1) + acc;
+    acc += cut[i];
+  }
+  if (t == kMetaThreads - 1)
+    num_splits[B] = used_before(cuts.last_at_or_before(W - 1) + 1) + inc;
 }
 
 }  // namespace
@@ -262,14 +397,19 @@ extern "C" int fa_mla_get_metadata(const int32_t* cache_seqlens, int32_t batch, 
   FA_CHECK_ARG(tile_md != nullptr && num_splits != nullptr, "output pointer is NULL");
   FA_CHECK_ARG(reinterpret_cast<uintptr_t>(tile_md) % 16 == 0, "tile_md is not 16-byte aligned");
   const bool small = num_parts <= fa::kMetaThreadsSmall && batch <= 4 * fa::kMetaThreadsSmall;
-  if (small) {
-    hipLaunchKernelGGL(fa::mla_metadata_kernel<fa::kMetaThreadsSmall>, dim3(1),
-                       dim3(fa::kMetaThreadsSmall), 0, static_cast<hipStream_t>(stream),
-                       cache_seqlens, batch, topk, num_parts, fixed_overhead, tile_md, num_splits);
+  const dim3 threads(small ? fa::kMetaThreadsSmall : fa::kMetaThreadsMax);
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const long long t = (static_cast<long long>(topk) + fa::kPage - 1) / fa::kPage;
+  if (topk > 0 && fixed_overhead == 0 && batch * t < (1ll << 30)) {
+    hipLaunchKernelGGL(small ? fa::mla_metadata_uniform_kernel<fa::kMetaThreadsSmall>
+                             : fa::mla_metadata_uniform_kernel<fa::kMetaThreadsMax>,
+                       dim3(1), threads, 0, s, batch, static_cast<int>(t), num_parts, tile_md,
+                       num_splits);
   } else {
-    hipLaunchKernelGGL(fa::mla_metadata_kernel<fa::kMetaThreadsMax>, dim3(1),
-                       dim3(fa::kMetaThreadsMax), 0, static_cast<hipStream_t>(stream),
-                       cache_seqlens, batch, topk, num_parts, fixed_overhead, tile_md, num_splits);
+    hipLaunchKernelGGL(small ? fa::mla_metadata_kernel<fa::kMetaThreadsSmall>
+                             : fa::mla_metadata_kernel<fa::kMetaThreadsMax>,
+                       dim3(1), threads, 0, s, cache_seqlens, batch, topk, num_parts,
+                       fixed_overhead, tile_md, num_splits);
   }
   FA_CHECK_HIP(hipGetLastError());
   return FA_OK;
