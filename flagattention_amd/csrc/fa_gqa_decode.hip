@@ -174,7 +174,8 @@ __global__ __launch_bounds__(kGThreads, D <= 128 ? 2 : 1) void gqa_decode_kernel
   const unsigned char* kp = static_cast<const unsigned char*>(a.k);
   const unsigned char* vp = static_cast<const unsigned char*>(a.v);
 
-  // Paged: the split's block-table slice goes to LDS first.  A page lookup is then an
+  // Paged, unless page ids come in pairs by scalar loads (below): the split's block-table
+  // slice goes to LDS first.  A page lookup is then an
   // LDS read; read from global memory it would be a vector load, and the wait for it
   // (vmcnt counts in order) would also wait for the previous tile's K/V loads, leaving
   // one tile in flight per wave.
@@ -184,8 +185,10 @@ __global__ __launch_bounds__(kGThreads, D <= 128 ? 2 : 1) void gqa_decode_kernel
   const int bs_shift = kPaged && a.block_size > 0 && (a.block_size & (a.block_size - 1)) == 0
                            ? __builtin_ctz(static_cast<unsigned int>(a.block_size))
                            : -1;
+  // see issue; nothing to stage then (0.3 us of a short call)
+  const bool page_pairs = kPaged && bs_shift >= 4 && (t0 & 15) == 0;
   if constexpr (kPaged) {
-    if (ntok > 0) {
+    if (ntok > 0 && !page_pairs) {
       blk_lo = t0 / a.block_size;
       const int nblk = (t1 - 1) / a.block_size - blk_lo + 1;
       tbl_lds = nblk <= kTblMax;
@@ -198,7 +201,7 @@ __global__ __launch_bounds__(kGThreads, D <= 128 ? 2 : 1) void gqa_decode_kernel
         }
       }
     }
-    __syncthreads();
+    if (!page_pairs) __syncthreads();  // uniform
   }
 
   // Q^T operand: row c16, dims 32kk + 8G..+7 (zeros past D or past the last row)
@@ -222,7 +225,6 @@ __global__ __launch_bounds__(kGThreads, D <= 128 ? 2 : 1) void gqa_decode_kernel
   // multiple of 16: each 16-token half of a tile lies in one page, so a tile needs two
   // page ids, wave-uniform.  They are fetched with scalar loads one tile ahead (the
   // wave's next tile is u + 4), so no load address of a tile waits on a lookup.
-  const bool page_pairs = kPaged && bs_shift >= 4 && (t0 & 15) == 0;
   const int32_t* const bt_row = kPaged ? a.block_table + static_cast<long long>(b) * a.bt_stride_b
                                        : nullptr;
   auto half_page = [&](int u, int h) -> int {  // page of tile u's half h, -1 if none

@@ -323,6 +323,9 @@ int64_t choose_splits(int64_t base, int64_t max_len, int64_t cus) {
   return std::max<int64_t>(1, std::min(cdiv(2 * cus, base), cdiv(max_len, kMinSplitTokens)));
 }
 
+// whole 32-key tiles (gqa.py)
+int64_t whole_tiles(int64_t tokens) { return cdiv(tokens, 32) * 32; }
+
 void run_gqa(fa_gqa_decode_args& a, int64_t rows, const c10::Device& device) {
   at::Tensor part;
   if (a.num_splits > 1) {
@@ -370,7 +373,8 @@ PyObject* paged(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (num_splits == 0) {
     const int cus = cu_count(device.index());
     if (cus == 0) return none();
-    split_tokens = cdiv(max_len, choose_splits(seqs * h_kv * cdiv(h_q / h_kv, 16), max_len, cus));
+    split_tokens = whole_tiles(
+        cdiv(max_len, choose_splits(seqs * h_kv * cdiv(h_q / h_kv, 16), max_len, cus)));
   } else if (num_splits == 1) {
     split_tokens = max_len;
   } else {
@@ -451,7 +455,7 @@ PyObject* contiguous(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   int64_t s = many && n <= 512
                   ? 1
                   : choose_splits(batch * h_kv * cdiv(rows, many ? 128 : 16), n, cus);
-  int64_t split_tokens = cdiv(n, s);
+  int64_t split_tokens = whole_tiles(cdiv(n, s));
   s = cdiv(n, split_tokens);
   if (s == 1) split_tokens = 1 << 30;
   at::Tensor out, lse;
