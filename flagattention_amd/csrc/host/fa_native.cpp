@@ -316,11 +316,16 @@ bool gqa_dtype(const at::Tensor& t) {
   return t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16;
 }
 
-constexpr int64_t kMinSplitTokens = 256;
-
-int64_t choose_splits(int64_t base, int64_t max_len, int64_t cus) {
-  if (base >= cus || max_len <= kMinSplitTokens) return 1;
-  return std::max<int64_t>(1, std::min(cdiv(2 * cus, base), cdiv(max_len, kMinSplitTokens)));
+// The split rule of gqa.py (choose_splits): rows = query rows per KV head, pairs = batch x KV
+// heads.
+int64_t choose_splits(int64_t pairs, int64_t rows, int64_t rows_per_wg, int64_t d, int64_t max_len,
+                      int64_t cus) {
+  const int64_t base = pairs * cdiv(rows, rows_per_wg);
+  if (base >= cus || max_len <= 256) return 1;
+  const int64_t s = std::min(cdiv(2 * cus, base), cdiv(max_len, 256));
+  const int64_t few = std::min(cdiv(cus, base), cdiv(max_len, 128));
+  if (few > (d > 64 ? 64 : 16) || pairs * rows * few * d > (int64_t{1} << 21)) return s;
+  return std::max(s, few);
 }
 
 // whole 32-key tiles (gqa.py)
@@ -374,7 +379,7 @@ PyObject* paged(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int cus = cu_count(device.index());
     if (cus == 0) return none();
     split_tokens = whole_tiles(
-        cdiv(max_len, choose_splits(seqs * h_kv * cdiv(h_q / h_kv, 16), max_len, cus)));
+        cdiv(max_len, choose_splits(seqs * h_kv, h_q / h_kv, 16, d, max_len, cus)));
   } else if (num_splits == 1) {
     split_tokens = max_len;
   } else {
@@ -454,7 +459,7 @@ PyObject* contiguous(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool many = (d == 64 || d == 128 || d == 256) && rows > 16;
   int64_t s = many && n <= 512
                   ? 1
-                  : choose_splits(batch * h_kv * cdiv(rows, many ? 128 : 16), n, cus);
+                  : choose_splits(batch * h_kv, rows, many ? 128 : 16, d, n, cus);
   int64_t split_tokens = whole_tiles(cdiv(n, s));
   s = cdiv(n, split_tokens);
   if (s == 1) split_tokens = 1 << 30;

@@ -37,6 +37,16 @@ HEAD_DIMS = (16, 32, 64, 128, 256, 512)
 ROWS_PER_WG = 16
 TILE_TOKENS = 32
 MIN_SPLIT_TOKENS = 256
+# Splits of one 32-key tile per wave where the launch is bound by the length of a work-group's
+# chain of tiles: 8 sequences of up to 1,000 tokens (32 heads of 4 KV heads, D = 128, paged)
+# 11.6 us a call in 4 splits, 10.5 in 8; one of 1,000 at D = 512 27.5 -> 17.7; 5 positions
+# x group 8 over 1,000 keys 11.6 -> 9.4.  Not once the CUs are full, and not where the combine
+# would take back what they give: above 64 splits (16 up to head dim 64; 4 heads over 20,000
+# keys, D = 64: 8.6 us in 79 splits, 9.3 in 157; over 4,000 7.7 in 16, 7.9 in 32) or above 2^21
+# partial values (4 x 128 positions, 8 heads, 900 keys: 17.8 us in 4 splits, 21.2 in 8).
+SHORT_SPLIT_TOKENS = 128
+MAX_SHORT_SPLITS = 64
+MAX_SHORT_PARTIALS = 1 << 21
 # The many-row kernel (csrc/fa_prefill.h): head dims, rows per KV head above which the
 # library uses it for contiguous K/V, and its rows per work-group.
 PREFILL_DIMS = (64, 128, 256)
@@ -77,14 +87,20 @@ def _cu_count(device: torch.device) -> int:
 
 
 def choose_splits(batch: int, h_kv: int, rows_per_kv_head: int, max_len: int,
-                  cu_count: int, rows_per_wg: int = ROWS_PER_WG) -> int:
+                  cu_count: int, rows_per_wg: int = ROWS_PER_WG, head_dim: int = 128) -> int:
     """Split-KV count: none when batch x KV heads x row blocks already gives every CU a
     work-group, else enough splits for about two work-groups per CU, each at least
-    MIN_SPLIT_TOKENS keys long."""
+    MIN_SPLIT_TOKENS keys long, or (few rows) for one per CU, each at least
+    SHORT_SPLIT_TOKENS."""
     base = batch * h_kv * -(-rows_per_kv_head // rows_per_wg)
     if base >= cu_count or max_len <= MIN_SPLIT_TOKENS:
         return 1
-    return max(1, min(-(-2 * cu_count // base), -(-max_len // MIN_SPLIT_TOKENS)))
+    s = min(-(-2 * cu_count // base), -(-max_len // MIN_SPLIT_TOKENS))
+    short = min(-(-cu_count // base), -(-max_len // SHORT_SPLIT_TOKENS))
+    if (short > (MAX_SHORT_SPLITS if head_dim > 64 else 16) or
+            batch * h_kv * rows_per_kv_head * short * head_dim > MAX_SHORT_PARTIALS):
+        return s
+    return max(s, short)
 
 
 def whole_tiles(tokens: int) -> int:
@@ -171,7 +187,8 @@ def paged_attention(
     device = query.device
     out = torch.empty_like(query)
     if num_splits == 0:
-        s = choose_splits(num_seqs, h_kv, h_q // h_kv, max_context_len, _cu_count(device))
+        s = choose_splits(num_seqs, h_kv, h_q // h_kv, max_context_len, _cu_count(device),
+                          head_dim=d)
         split_tokens = whole_tiles(-(-max_context_len // s))
     elif num_splits == 1:
         split_tokens = max_context_len
@@ -229,7 +246,7 @@ def _dense_decode(q, k, v, causal, sm_scale, want_lse):
     many = d in PREFILL_DIMS and rows > PREFILL_MIN_ROWS
     s = (1 if many and n <= PREFILL_UNSPLIT_TOKENS
          else choose_splits(batch, h_kv, rows, n, _cu_count(device),
-                            PREFILL_ROWS_PER_WG if many else ROWS_PER_WG))
+                            PREFILL_ROWS_PER_WG if many else ROWS_PER_WG, d))
     split_tokens = whole_tiles(-(-n // s)) if n > 0 else 1
     s = max(1, -(-n // split_tokens)) if n > 0 else 1
     if s == 1:

@@ -210,6 +210,22 @@ def test_paged_attention_odd_block_sizes(block_size, group, num_splits):
                          seed=block_size * 10 + group + num_splits)
 
 
+@pytest.mark.parametrize("seqs,h_kv,group,D,block_size,max_len", [
+    (1, 1, 8, 128, 16, 257),    # 3 splits of 96, the last of 65 keys
+    (3, 2, 4, 64, 16, 385),
+    (1, 4, 4, 512, 16, 1000),
+    (2, 2, 1, 256, 32, 1025),
+    (1, 1, 4, 128, 16, 8192),   # 64 splits, the most
+])
+def test_paged_attention_short_splits(seqs, h_kv, group, D, block_size, max_len):
+    """Splits of 128 keys (one tile per wave), which few work-groups take on their own."""
+    from flagattention_amd import gqa
+    need_gpu()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert gqa.choose_splits(seqs, h_kv, group, max_len, cus, head_dim=D) == -(-max_len // 128)
+    base_paged_attention(seqs, h_kv * group, group, D, block_size, max_len, 0, seed=max_len)
+
+
 def _oracle_chunked(q, k, v, causal, upcast, chunk=4):
     """flash_attention_ref over batch slices (the GQA repeat of a whole batch would not fit
     in host memory at these shapes)."""

@@ -55,6 +55,9 @@ def _same(a, b):
     (1, 4, 2, 1, 700, 64, False, None, "bhtd"),    # split, 16-row kernel
     (2, 8, 1, 3, 300, 128, True, 0.2, "bthd"),     # 24 rows, unsplit
     (2, 8, 1, 3, 3000, 128, True, -1, "bthd"),     # 24 rows, split
+    (4, 8, 8, 128, 900, 128, True, None, "bthd"),  # too many partial values for short splits
+    (1, 4, 1, 1, 4000, 64, False, None, "bhtd"),   # too many short splits at head dim 64
+    (1, 4, 1, 1, 8193, 128, False, None, "bhtd"),  # and at 128
     (1, 2, 2, 200, 2000, 256, True, None, "bhtd"),
     (1, 2, 2, 5, 40, 32, False, None, "bthd"),
     (1, 1, 1, 2, 900, 512, True, None, "bhtd"),
