@@ -328,6 +328,13 @@ int64_t choose_splits(int64_t pairs, int64_t rows, int64_t rows_per_wg, int64_t 
   return std::max(s, few);
 }
 
+// Whether a many-row call of few keys runs unsplit (gqa.py, prefill_unsplit).
+bool prefill_unsplit(int64_t pairs, int64_t rows, int64_t d, int64_t n, int64_t cus) {
+  if (n > 512) return false;
+  const int64_t few = std::min(cdiv(cus, pairs * cdiv(rows, 128)), cdiv(n, 128));
+  return n <= (d == 256 ? 256 : 384) || few < 3 || pairs * rows * few * d > (int64_t{1} << 20);
+}
+
 // whole 32-key tiles (gqa.py)
 int64_t whole_tiles(int64_t tokens) { return cdiv(tokens, 32) * 32; }
 
@@ -457,7 +464,7 @@ PyObject* contiguous(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   // the row counts and split rule of gqa.py
   const int64_t rows = h_q / h_kv * m;
   const bool many = (d == 64 || d == 128 || d == 256) && rows > 16;
-  int64_t s = many && n <= 512
+  int64_t s = many && prefill_unsplit(batch * h_kv, rows, d, n, cus)
                   ? 1
                   : choose_splits(batch * h_kv, rows, many ? 128 : 16, d, n, cus);
   int64_t split_tokens = whole_tiles(cdiv(n, s));

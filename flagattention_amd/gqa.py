@@ -52,10 +52,14 @@ MAX_SHORT_PARTIALS = 1 << 21
 PREFILL_DIMS = (64, 128, 256)
 PREFILL_MIN_ROWS = 16
 PREFILL_ROWS_PER_WG = 128
-# Up to here the second launch costs more than the keys it saves a work-group: a 300-token
-# prompt (8 KV heads, D = 128) takes 18.7 us unsplit, 25.4 us in two splits; at 2,000 keys
-# (D = 256, 4 KV heads) 8 splits take 27.9 us, 4 of them 36.4 us.
+# Up to 512 keys the many-row kernel splits only where at least 3 short splits leave at most
+# 2^20 partial values, and there from 385 keys (257 at head dim 256, whose tiles are half as
+# long): otherwise the second launch costs more than the keys it saves a work-group.  Per call,
+# unsplit / split: 5 positions x group 4 over 500 keys (8 KV heads, D = 128) 13.5 / 8.8 us, 4 x 8
+# over 300 at D = 256 21.3 / 12.6; but a 300-token prompt at D = 128 10.7 / 12.8, at D = 64 8.0 /
+# 10.3, and 100 x 4 over 400 keys (1.6 million partial values) 13.8 / 14.8.
 PREFILL_UNSPLIT_TOKENS = 512
+PREFILL_MAX_PARTIALS = 1 << 20
 
 # Benchmark hook: a (start, end) pair of CUDA events recorded on the launch stream right
 # around the next decode kernel launch (not the combine); cleared after that launch.
@@ -101,6 +105,17 @@ def choose_splits(batch: int, h_kv: int, rows_per_kv_head: int, max_len: int,
             batch * h_kv * rows_per_kv_head * short * head_dim > MAX_SHORT_PARTIALS):
         return s
     return max(s, short)
+
+
+def prefill_unsplit(batch: int, h_kv: int, rows: int, n: int, cu_count: int,
+                    head_dim: int) -> bool:
+    """Whether a many-row call of few keys runs unsplit (see PREFILL_UNSPLIT_TOKENS)."""
+    if n > PREFILL_UNSPLIT_TOKENS:
+        return False
+    short = min(-(-cu_count // (batch * h_kv * -(-rows // PREFILL_ROWS_PER_WG))),
+                -(-n // SHORT_SPLIT_TOKENS))
+    return (n <= (256 if head_dim == 256 else 384) or short < 3 or
+            batch * h_kv * rows * short * head_dim > PREFILL_MAX_PARTIALS)
 
 
 def whole_tiles(tokens: int) -> int:
@@ -244,8 +259,9 @@ def _dense_decode(q, k, v, causal, sm_scale, want_lse):
     lse = torch.empty((batch, h_q, m), dtype=torch.float32, device=device) if want_lse else None
     rows = (h_q // h_kv) * m
     many = d in PREFILL_DIMS and rows > PREFILL_MIN_ROWS
-    s = (1 if many and n <= PREFILL_UNSPLIT_TOKENS
-         else choose_splits(batch, h_kv, rows, n, _cu_count(device),
+    cus = _cu_count(device)
+    s = (1 if many and prefill_unsplit(batch, h_kv, rows, n, cus, d)
+         else choose_splits(batch, h_kv, rows, n, cus,
                             PREFILL_ROWS_PER_WG if many else ROWS_PER_WG, d))
     split_tokens = whole_tiles(-(-n // s)) if n > 0 else 1
     s = max(1, -(-n // split_tokens)) if n > 0 else 1

@@ -386,6 +386,8 @@ def _laid_out(x, form):
     (2, 4, 4, 127, 127, True, "odd"),     # realigned by a copy, short of a tile
     (8, 16, 8, 300, 193, True, "bthd"),   # M > N, every work-group resident at once
     (1, 4, 2, 40, 2100, True, "padded"),  # splits, the last one ragged
+    (1, 8, 2, 5, 385, True, "bhtd"),      # short splits of few keys, the last of one key
+    (2, 8, 1, 4, 257, False, "bthd"),     # at head dim 256 already here, unsplit otherwise
     (3, 3, 1, 200, 1600, False, "bhtd"),  # a batch that is not a multiple of the XCDs
 ])
 def test_flash_attention_many_rows(D, B, Hq, Hk, M, N, causal, form):

@@ -56,6 +56,10 @@ def _same(a, b):
     (2, 8, 1, 3, 300, 128, True, 0.2, "bthd"),     # 24 rows, unsplit
     (2, 8, 1, 3, 3000, 128, True, -1, "bthd"),     # 24 rows, split
     (4, 8, 8, 128, 900, 128, True, None, "bthd"),  # too many partial values for short splits
+    (1, 8, 2, 5, 385, 128, True, None, "bhtd"),    # few keys, short splits
+    (1, 8, 2, 5, 384, 128, True, None, "bhtd"),    # one key fewer: unsplit
+    (2, 4, 1, 9, 257, 256, False, None, "bthd"),   # head dim 256 from 257
+    (1, 8, 8, 400, 512, 128, True, None, "bthd"),  # too many partial values: unsplit
     (1, 4, 1, 1, 4000, 64, False, None, "bhtd"),   # too many short splits at head dim 64
     (1, 4, 1, 1, 8193, 128, False, None, "bhtd"),  # and at 128
     (1, 2, 2, 200, 2000, 256, True, None, "bhtd"),
