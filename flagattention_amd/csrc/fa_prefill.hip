@@ -162,8 +162,11 @@ __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_
   const int lim = limit_of(row);
 
   const float ninf = -__builtin_inff();
-  const float scale_log2 = fabsf(a.scale) * kLog2e;
-  const bool negate = a.scale < 0.f;  // uniform
+  // The scale is applied inside the exponent, after the mask and the maximum.  That needs a
+  // positive one: a negative one turns the order of the scores, and 0 times a masked -inf is
+  // NaN.  Otherwise the scores are scaled before either (prescale).
+  const bool prescale = !(a.scale > 0.f);  // uniform
+  const float scale_log2 = prescale ? 1.f : a.scale * kLog2e;
 
   const unsigned char* const kp = static_cast<const unsigned char*>(a.k) +
                                   2 * (b * a.k_stride_0 + hk * a.k_stride_h);
@@ -261,11 +264,11 @@ __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_
       for (int tt = 0; tt < kSub; ++tt) s[tt] = mfma_32x32x16(ka[kk & 1][tt], qf[kk], s[tt]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (negate) {
+    if (prescale) {
 #pragma unroll
       for (int tt = 0; tt < kSub; ++tt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[tt][i] = -s[tt][i];
+        for (int i = 0; i < 16; ++i) s[tt][i] *= a.scale * kLog2e;
     }
     if (start + kTok > wave_min) {  // uniform: some row does not see the whole tile
       const int left = lim - start - 4 * g;

@@ -423,3 +423,21 @@ def test_flash_attention_many_rows_late_maximum():
     torch.cuda.synchronize()
     assert_lowp_rule(o.cpu(), o_ref, o_low)
     assert float((lse.cpu() - lse_ref).abs().max()) <= 1e-3
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("M, N", [(40, 100), (17, 2100)])  # ragged tiles; short and long splits
+def test_flash_attention_many_rows_scale_zero(D, M, N):
+    """sm_scale 0 weighs every visible key alike, also where a tile has masked keys (0 times
+    a masked score must not become NaN): out is the mean of the visible V rows, lse the log of
+    their number."""
+    need_gpu()
+    for dtype, causal, scale in ((torch.float16, True, 0.0), (torch.bfloat16, False, -0.0)):
+        q, k, v = _splitkv_inputs(1, 2, 1, M, N, D, dtype, "BHTD", 1.0, D + N)
+        o_ref, lse_ref = go.flash_attention_ref(q, k, v, causal, sm_scale=scale, upcast=True)
+        o_low, _ = go.flash_attention_ref(q, k, v, causal, sm_scale=scale, upcast=False)
+        o, lse, _, _, _ = flag_attn.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), causal, scale,
+                                                    return_log_normalizer=True)
+        torch.cuda.synchronize()
+        assert_lowp_rule(o.cpu(), o_ref, o_low)
+        assert float((lse.cpu() - lse_ref).abs().max()) <= 1e-5  # log of a number up to 2,100
