@@ -52,6 +52,12 @@ constexpr int kPWaves = 4;
 constexpr int kPThreads = 64 * kPWaves;
 constexpr int kPWaveRows = 32;
 static_assert(kPWaves * kPWaveRows == kPrefillRows, "rows per work-group");
+// A row's reference is the rounded product of its largest score and the scale; the fused
+// multiply-add of the exponents does not round that product, which leaves the largest
+// exponent at the rounding error instead of 0: up to 2^-15 for references below 2^10 (P still
+// rounds to 1), but +-32 at 2^30.  Past this reference the scores are scaled in a pass of their
+// own.
+constexpr float kFusedScale = 1024.f;
 
 template <typename T>
 struct PVec {
@@ -297,6 +303,14 @@ __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_
         for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
     }
     const float nm = mref == ninf ? 0.f : -mref;
+    float c = scale_log2;
+    if (__ballot(fabsf(nm) > kFusedScale) != 0ull) {  // uniform
+#pragma unroll
+      for (int tt = 0; tt < kSub; ++tt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[tt][i] *= c;
+      c = 1.f;
+    }
     T8 pb[kPSteps];
     float ps = 0.f;
 #pragma unroll
@@ -304,7 +318,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float p = __builtin_amdgcn_exp2f(
-            __builtin_fmaf(s[ss >> 1][8 * (ss & 1) + i], scale_log2, nm));
+            __builtin_fmaf(s[ss >> 1][8 * (ss & 1) + i], c, nm));
         ps += p;
         pb[ss][i] = static_cast<T>(p);
       }

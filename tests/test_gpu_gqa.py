@@ -441,3 +441,36 @@ def test_flash_attention_many_rows_scale_zero(D, M, N):
         torch.cuda.synchronize()
         assert_lowp_rule(o.cpu(), o_ref, o_low)
         assert float((lse.cpu() - lse_ref).abs().max()) <= 1e-5  # log of a number up to 2,100
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("dtype, amp", [
+    (torch.float16, 30.0),       # largest scores of about 2^12 in log2 units
+    (torch.float16, 300.0),      # of 2^19
+    (torch.float16, 10000.0),    # of 2^29: their rounding alone is past fp16's range
+    (torch.bfloat16, 300000.0),  # of 2^39, and past bf16's
+])
+def test_flash_attention_many_rows_large_scores(D, dtype, amp):
+    """Scores far apart: the largest takes all the weight.  Its exponent has to be 0 whatever
+    the size of the scores, so that out is its V row to the bit and lse the score itself."""
+    need_gpu()
+    for causal, sign, N in ((True, 1, 700), (False, 1, 2100), (False, -1, 300)):
+        q, k, v = _splitkv_inputs(1, 2, 1, 40, N, D, torch.float32, "BHTD", 1.0, D + N)
+        q, k, v = (amp * q).to(dtype), (amp * k).to(dtype), v.to(dtype)
+        scale = sign * D ** -0.5
+        s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) * scale
+        if causal:
+            s = s.masked_fill(~torch.ones(40, N, dtype=torch.bool).tril(N - 40), float("-inf"))
+        top, at = s.topk(2, dim=-1)
+        # rows whose two best scores an fp32 sum over D products, with its scale, tells apart
+        # by the 40 that leave e^-40 to all others
+        size = (q.double().norm(dim=-1) * k.double().norm(dim=-1).max() * abs(scale))
+        clear = top[..., 0] - top[..., 1] > 40 + (D + 2) * 2.0 ** -23 * size
+        assert float(clear.float().mean()) > 0.5  # most rows count
+        o, lse, _, _, _ = flag_attn.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), causal, scale,
+                                                    return_log_normalizer=True)
+        torch.cuda.synchronize()
+        want = v[0, 0][at[..., 0]]
+        assert torch.equal(o.cpu()[clear], want[clear])
+        err = (lse.cpu().double() - top[..., 0]).abs()
+        assert bool((err <= (D + 2) * 2.0 ** -23 * size)[clear].all())
