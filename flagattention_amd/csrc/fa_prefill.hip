@@ -18,10 +18,14 @@
 //     whole kernel;
 //   softmax: a lane holds half of one row's scores (lane % 32 = row, the other half is 32
 //     lanes away), so the row max is in-lane plus one lane swap, and the row sum stays
-//     in-lane until the end.  A tile in which no row of the wave has a new maximum skips the
-//     rescale.  (Letting P grow to 2^6 before rescaling was 5% faster, but then a row's
-//     largest P is no longer exactly 1 and its rounding to 16 bits shows: error against 64
-//     bits 2.30e-3 instead of 2.17e-3, the 16-row kernel's is 2.08e-3.)
+//     in-lane until the end.  The reference that P is relative to follows each tile's
+//     maximum, down as well as up (kFall), and the accumulators are rescaled at every tile:
+//     the largest P of a tile is then exactly 1, and its rounding to 16 bits costs nothing.
+//     With one running maximum instead (rescaling only where some row has a new one) a long
+//     row has few such keys: 2% faster, but bf16 error against 64 bits 2.26e-3 instead of
+//     2.09e-3 at the first shape below, where the 16-row kernel (a reference per 32-key tile
+//     and wave) has 2.20e-3.  Over few keys the tile's halves take a reference each
+//     (kHalvesKeys).
 //   O^T[D, 32 rows] += V^T P^T: P^T (B) is the lane's own scores rounded to 16 bits (the
 //     k order only has to agree between A and B: lane half g holds keys 16s + 4g..+3 and
 //     16s + 8 + 4g..+3 of k-step s), V^T (A) by the transposing ds_read_b64_tr_b16.
@@ -30,10 +34,10 @@
 // read one k-step ahead of their MFMAs (2% at D = 128, 8% at D = 256 causal).
 //
 // Measured (bf16, wall time per call, 16-row kernel -> this one): 2,048 new positions behind
-// 1,901, B = 2, 32 heads of 8 KV heads, D = 128, causal: 1578 -> 220 us (0.89 PFLOP/s; a
+// 1,901, B = 2, 32 heads of 8 KV heads, D = 128, causal: 1578 -> 213 us (0.92 PFLOP/s; a
 // large bf16 matrix product reaches 1.4 here, and the socket's power limit bounds both);
-// 8 positions x group 8 over 2,000 keys, B = 8: 50 -> 25 us (then bound by the host);
-// 5 positions x group 4 over 4,000 keys, B = 8: 59 -> 27 us.
+// 8 positions x group 8 over 2,000 keys, B = 8: 45 -> 23 us;
+// 5 positions x group 4 over 4,000 keys, B = 8: 59 -> 26 us.
 //
 // LDS layouts (16-byte chunk c of token row r): K at chunk c ^ fk(r), so that the 16 rows
 // of a quarter wave's reads at one chunk cover 256 distinct bytes; V at pair (c / 2) ^
@@ -58,6 +62,17 @@ static_assert(kPWaves * kPWaveRows == kPrefillRows, "rows per work-group");
 // rounds to 1), but +-32 at 2^30.  Past this reference the scores are scaled in a pass of their
 // own.
 constexpr float kFusedScale = 1024.f;
+// How far below a row's running maximum (log2 units) its reference may fall: the sums grow by
+// at most 2^4 over those of one running maximum.  Error at the first shape above 2.11e-3 at 2,
+// 2.090e-3 at 4 and at 8.
+constexpr float kFall = 4.f;
+// Up to this many keys that a row sees on average, the 32-key halves of a 64-key tile take a
+// reference each.  bf16 error against 64 bits, 16-row kernel / tile / halves: 300 keys
+// 2.056e-3 / 2.115e-3 / 2.042e-3, 300 x 300 causal 1.900e-3 / 1.924e-3 / 1.894e-3, 1,024 x
+// 1,024 causal 1.946e-3 / 1.963e-3 / 1.924e-3; at 2,100 keys 2.087e-3 / 2.076e-3 / 2.015e-3,
+// 3,000 x 3,000 causal 1.987e-3 / 1.985e-3 / 1.942e-3.  The second rescale costs 5 .. 9%
+// (1,024 x 1,024 37.4 -> 40.7 us), so it stays off where the tile's maximum is enough.
+constexpr int kHalvesKeys = 1536;
 
 template <typename T>
 struct PVec {
@@ -99,7 +114,7 @@ __device__ inline int fv(int r) {
   return C >= 16 ? (((r & 3) << 1) | ((r >> 2) & 1)) : ((r & 2) | ((r >> 2) & 1));
 }
 
-template <typename T, int D>
+template <typename T, int D, bool kHalves>
 __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_decode_args a,
                                                                   const int n_rb,
                                                                   const int fits) {
@@ -109,12 +124,13 @@ __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_
   constexpr int kRowB = 2 * D;           // bytes per token row
   constexpr int kTok = D <= 128 ? 64 : 32;  // keys per tile
   constexpr int kSub = kTok / 32;        // 32-key sub-tiles of S^T
+  constexpr int kParts = kHalves ? kSub : 1;  // softmax references per tile
+  constexpr int kPer = kSub / kParts;    // sub-tiles of each
   constexpr int kTileB = kTok * kRowB;
   constexpr int kCopies = kTileB / 1024 / kPWaves;  // 1 KB copies per wave, of K and of V
   constexpr int kRowsPerCopy = 1024 / kRowB;
   constexpr int kKSteps = D / 16;        // MFMA k-steps of QK
   constexpr int kDimTiles = D / 32;      // 32-dim tiles of O^T
-  constexpr int kPSteps = kTok / 16;     // MFMA k-steps of PV
   static_assert(kCopies * kPWaves * 1024 == kTileB, "whole copies per wave");
   // [K, V][tile parity]; the epilogue stages each wave's 32 output rows over them
   __shared__ __attribute__((aligned(16))) unsigned char bufs[4 * kTileB];
@@ -225,15 +241,16 @@ __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_
   floatx16 acc[kDimTiles];
 #pragma unroll
   for (int dt = 0; dt < kDimTiles; ++dt) acc[dt] = floatx16{};
-  float mref = ninf, lsum = 0.f;
+  float mref = ninf, mrun = ninf, lsum = 0.f;
 
   // lane offsets of the LDS reads
   const int kbase = c32 * kRowB + 16 * (g ^ fk<C>(c32));  // chunk 2kk + g: xor 32 kk
   const int h16 = lane >> 4, e = (lane & 15) >> 2, qd = lane & 3;
   const int vtok = 4 * g + e;  // token within 8
-  int vbase[kDimTiles];
+  constexpr int kVBases = kDimTiles < 4 ? kDimTiles : 4;  // fv < 8: dt + 4 is 256 bytes on
+  int vbase[kVBases];
 #pragma unroll
-  for (int dt = 0; dt < kDimTiles; ++dt)
+  for (int dt = 0; dt < kVBases; ++dt)
     vbase[dt] = vtok * kRowB + 32 * ((2 * dt + (h16 & 1)) ^ fv<C>(vtok)) + 16 * (qd >> 1) +
                 8 * (qd & 1);
 
@@ -286,14 +303,18 @@ __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_
           s[tt][i] = j < left ? s[tt][i] : ninf;
         }
     }
-    float mx = s[0][0];
+    // softmax and PV of the tile, or of its 32-key halves one after the other
 #pragma unroll
-    for (int tt = 0; tt < kSub; ++tt)
+    for (int part = 0; part < kParts; ++part) {
+      const int tt0 = part * kPer;
+      float mx = s[tt0][0];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[tt][i]);
-    mx = max_xor32(mx) * scale_log2;
-    if (__ballot(mx > mref) != 0ull) {  // uniform
-      const float m_new = fmaxf(mref, mx);
+      for (int tt = tt0; tt < tt0 + kPer; ++tt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[tt][i]);
+      mx = max_xor32(mx) * scale_log2;
+      mrun = fmaxf(mrun, mx);
+      const float m_new = fmaxf(mx, mrun - kFall);
       const float alpha = m_new == ninf ? 1.f : __builtin_amdgcn_exp2f(mref - m_new);
       lsum *= alpha;
       mref = m_new;
@@ -301,38 +322,38 @@ __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_
       for (int dt = 0; dt < kDimTiles; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
-    }
-    const float nm = mref == ninf ? 0.f : -mref;
-    float c = scale_log2;
-    if (__ballot(fabsf(nm) > kFusedScale) != 0ull) {  // uniform
+      const float nm = mref == ninf ? 0.f : -mref;
+      float c = scale_log2;
+      if (__ballot(fabsf(nm) > kFusedScale) != 0ull) {  // uniform
 #pragma unroll
-      for (int tt = 0; tt < kSub; ++tt)
+        for (int tt = tt0; tt < tt0 + kPer; ++tt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[tt][i] *= c;
-      c = 1.f;
-    }
-    T8 pb[kPSteps];
-    float ps = 0.f;
-#pragma unroll
-    for (int ss = 0; ss < kPSteps; ++ss)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float p = __builtin_amdgcn_exp2f(
-            __builtin_fmaf(s[ss >> 1][8 * (ss & 1) + i], c, nm));
-        ps += p;
-        pb[ss][i] = static_cast<T>(p);
+          for (int i = 0; i < 16; ++i) s[tt][i] *= c;
+        c = 1.f;
       }
-    lsum += ps;
+      T8 pb[2 * kPer];
+      float ps = 0.f;
 #pragma unroll
-    for (int ss = 0; ss < kPSteps; ++ss)
+      for (int ss = 0; ss < 2 * kPer; ++ss)
 #pragma unroll
-      for (int dt = 0; dt < kDimTiles; ++dt) {
-        const unsigned char* const p = vb + 16 * ss * kRowB + vbase[dt];
-        const T4 lo = lds_tr_read4<T>(p);
-        const T4 hi = lds_tr_read4<T>(p + 8 * kRowB);
-        const T8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        acc[dt] = mfma_32x32x16(va, pb[ss], acc[dt]);
-      }
+        for (int i = 0; i < 8; ++i) {
+          const float p = __builtin_amdgcn_exp2f(
+              __builtin_fmaf(s[tt0 + (ss >> 1)][8 * (ss & 1) + i], c, nm));
+          ps += p;
+          pb[ss][i] = static_cast<T>(p);
+        }
+      lsum += ps;
+#pragma unroll
+      for (int ss = 0; ss < 2 * kPer; ++ss)
+#pragma unroll
+        for (int dt = 0; dt < kDimTiles; ++dt) {
+          const unsigned char* const p = vb + 16 * (2 * tt0 + ss) * kRowB + 256 * (dt >> 2) + vbase[dt & 3];
+          const T4 lo = lds_tr_read4<T>(p);
+          const T4 hi = lds_tr_read4<T>(p + 8 * kRowB);
+          const T8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+          acc[dt] = mfma_32x32x16(va, pb[ss], acc[dt]);
+        }
+    }
   }
   wait_vmem<0>();
   barrier();  // the tile buffers are free
@@ -398,12 +419,17 @@ void launch_prefill_t(const fa_gqa_decode_args* a, hipStream_t stream) {
                   static_cast<unsigned>(a->num_splits));
   // resident work-groups: 2 per CU (LDS), 4 at head dim 64 (VGPRs), 256 CUs
   const int fits = a->causal && a->num_splits == 1 && grid.x <= (a->d == 64 ? 1024u : 512u);
+  // device lengths are not known here: halves
+  const bool halves = a->seqlens || a->n - (a->causal ? a->m / 2 : 0) <= kHalvesKeys;
   if (a->d == 64)
-    hipLaunchKernelGGL((gqa_prefill_kernel<T, 64>), grid, dim3(kPThreads), 0, stream, *a, n_rb, fits);
+    hipLaunchKernelGGL((halves ? gqa_prefill_kernel<T, 64, true> : gqa_prefill_kernel<T, 64, false>),
+                       grid, dim3(kPThreads), 0, stream, *a, n_rb, fits);
   else if (a->d == 128)
-    hipLaunchKernelGGL((gqa_prefill_kernel<T, 128>), grid, dim3(kPThreads), 0, stream, *a, n_rb, fits);
+    hipLaunchKernelGGL((halves ? gqa_prefill_kernel<T, 128, true> : gqa_prefill_kernel<T, 128, false>),
+                       grid, dim3(kPThreads), 0, stream, *a, n_rb, fits);
   else
-    hipLaunchKernelGGL((gqa_prefill_kernel<T, 256>), grid, dim3(kPThreads), 0, stream, *a, n_rb, fits);
+    hipLaunchKernelGGL((gqa_prefill_kernel<T, 256, false>), grid, dim3(kPThreads), 0, stream, *a,
+                       n_rb, fits);
 }
 
 }  // namespace

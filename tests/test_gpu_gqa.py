@@ -474,3 +474,27 @@ def test_flash_attention_many_rows_large_scores(D, dtype, amp):
         assert torch.equal(o.cpu()[clear], want[clear])
         err = (lse.cpu().double() - top[..., 0]).abs()
         assert bool((err <= (D + 2) * 2.0 ** -23 * size)[clear].all())
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("N", [100, 500, 1536, 2100])  # both sides of the halves rule
+def test_flash_attention_many_rows_error(D, N):
+    """64 query rows at once are as close to the 64-bit result as 16 rows at a time (the 16-row
+    kernel; 256 pairs, so neither splits).  Both round P and the output to 16 bits, errors that
+    are independent from key to key: over a million output values their 2-norm varies by under
+    0.1%, a reference that leaves more of the large P inexact adds 1% to 6%."""
+    need_gpu()
+    for dtype in (torch.bfloat16, torch.float16):
+        gen = torch.Generator(device=DEV).manual_seed(D + N)
+        q, k, v = (torch.randn((4, 64, t, D), device=DEV, generator=gen).to(dtype)
+                   for t in (64, N, N))
+        many = flag_attn.flash_attention(q, k, v)
+        few = torch.cat([flag_attn.flash_attention(c, k, v) for c in q.split(16, dim=2)], dim=2)
+        err = {"many": 0.0, "few": 0.0}
+        for b in range(4):
+            s = torch.matmul(q[b].double(), k[b].double().transpose(1, 2).contiguous()) * D ** -0.5
+            exact = torch.matmul(torch.softmax(s, dim=-1), v[b].double())
+            for name, o in (("many", many), ("few", few)):
+                err[name] += float((o[b].double() - exact).square().sum())
+        say(f"D={D} N={N} {dtype}: many / few {(err['many'] / err['few']) ** 0.5:.4f}")
+        assert err["many"] <= 1.005 ** 2 * err["few"]
