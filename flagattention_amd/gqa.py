@@ -93,11 +93,11 @@ def _cu_count(device: torch.device) -> int:
 def choose_splits(batch: int, h_kv: int, rows_per_kv_head: int, max_len: int,
                   cu_count: int, rows_per_wg: int = ROWS_PER_WG, head_dim: int = 128) -> int:
     """Split-KV count: none when batch x KV heads x row blocks already gives every CU a
-    work-group, else enough splits for about two work-groups per CU, each at least
-    MIN_SPLIT_TOKENS keys long, or (few rows) for one per CU, each at least
-    SHORT_SPLIT_TOKENS."""
+    work-group (or there is nothing to launch: the library then raises), else enough splits
+    for about two work-groups per CU, each at least MIN_SPLIT_TOKENS keys long, or (few rows)
+    for one per CU, each at least SHORT_SPLIT_TOKENS."""
     base = batch * h_kv * -(-rows_per_kv_head // rows_per_wg)
-    if base >= cu_count or max_len <= MIN_SPLIT_TOKENS:
+    if base == 0 or base >= cu_count or max_len <= MIN_SPLIT_TOKENS:
         return 1
     s = min(-(-2 * cu_count // base), -(-max_len // MIN_SPLIT_TOKENS))
     short = min(-(-cu_count // base), -(-max_len // SHORT_SPLIT_TOKENS))
@@ -110,10 +110,10 @@ def choose_splits(batch: int, h_kv: int, rows_per_kv_head: int, max_len: int,
 def prefill_unsplit(batch: int, h_kv: int, rows: int, n: int, cu_count: int,
                     head_dim: int) -> bool:
     """Whether a many-row call of few keys runs unsplit (see PREFILL_UNSPLIT_TOKENS)."""
-    if n > PREFILL_UNSPLIT_TOKENS:
-        return False
-    short = min(-(-cu_count // (batch * h_kv * -(-rows // PREFILL_ROWS_PER_WG))),
-                -(-n // SHORT_SPLIT_TOKENS))
+    base = batch * h_kv * -(-rows // PREFILL_ROWS_PER_WG)
+    if base == 0 or n > PREFILL_UNSPLIT_TOKENS:
+        return base == 0
+    short = min(-(-cu_count // base), -(-n // SHORT_SPLIT_TOKENS))
     return (n <= (256 if head_dim == 256 else 384) or short < 3 or
             batch * h_kv * rows * short * head_dim > PREFILL_MAX_PARTIALS)
 

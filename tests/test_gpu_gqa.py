@@ -498,3 +498,20 @@ def test_flash_attention_many_rows_error(D, N):
                 err[name] += float((o[b].double() - exact).square().sum())
         say(f"D={D} N={N} {dtype}: many / few {(err['many'] / err['few']) ** 0.5:.4f}")
         assert err["many"] <= 1.005 ** 2 * err["few"]
+
+
+@pytest.mark.parametrize("B, M, N", [(0, 40, 100), (0, 40, 500), (0, 1, 100), (0, 1, 3000),
+                                     (0, 40, 3000), (2, 0, 100), (2, 0, 3000)])
+def test_empty_batch_or_query_is_the_librarys_argument_error(B, M, N):
+    """No sequence or no query position: the library's argument check answers, whatever the
+    number of keys (no split rule divides by the empty extent before it)."""
+    need_gpu()
+    q, k = (torch.zeros((B, h, t, 64), dtype=torch.float16, device=DEV) for h, t in ((4, M), (2, N)))
+    for call in (flag_attn.flash_attention, flag_attn.flash_attention_split_kv):
+        with pytest.raises(RuntimeError, match="must be >= 1"):
+            call(q, k, k)
+    if M == 1:
+        lens = torch.zeros((0,), dtype=torch.int32, device=DEV)
+        cache = torch.zeros((4, 2, 16, 64), dtype=torch.float16, device=DEV)
+        with pytest.raises(RuntimeError, match="must be >= 1"):
+            flag_attn.paged_attention(q[:, :, 0], cache, cache, lens, lens.new_zeros((0, 8)), 1.0, N)
