@@ -967,7 +967,8 @@ __global__ __launch_bounds__(kThreads, 1) void mla_decode_kernel(const fa_mla_de
       }
       barrier();
       unsigned int* const flags = reinterpret_cast<unsigned int*>(sm.p + 4096);
-      if (lane == 0) flags[wave] = __any(overflow) ? 1u : 0u;
+      const bool any = __any(overflow);  // over all lanes, so outside the branch
+      if (lane == 0) flags[wave] = any ? 1u : 0u;
       barrier();
       if ((flags[0] | flags[1] | flags[2] | flags[3]) == 0u) break;
 #pragma unroll

@@ -254,6 +254,37 @@ def test_sparse_fp8_wide_score_spread():
     assert_close(out, lse, ref_out, ref_lse, low, low_lse)
 
 
+@pytest.mark.parametrize("h_q,head", [(48, 5), (48, 47), (128, 30), (144, 139)])
+@pytest.mark.parametrize("mode", ["dense", "sparse", "fp8"])
+def test_wide_score_spread_of_one_row(h_q, head, mode):
+    """One row alone, and not the first of its 16-row tile, scores 180 log2 units above its
+    first tile's maximum: the work-group takes the second pass for it too (P would overflow
+    past 128)."""
+    need_gpu()
+    lens = [3000]
+    q, kc, bt, ld = orc.make_dense_inputs(1, h_q, 1, lens, seed=83, scale=0.1)
+    q[:, :, head] = 2.0
+    idx = orc.make_sparse_indices(1, 1, 1024, lens, seed=84, invalid_frac=0.0)
+    j = int(idx[0, 0, 900])  # a late tile, in any mode
+    if mode == "fp8":
+        kc = orc.make_fp8_cache(kc.shape[0], seed=85, lat_scale=0.1)
+        row = orc.fp8_rows_quantize(torch.full((1, 512), 1.5),
+                                    torch.full((1, 64), 1.5, dtype=torch.bfloat16),
+                                    torch.ones((1, 4)))
+        kc[int(bt[0, j // 64]), j % 64, 0, :] = row[0]
+    else:
+        _plant_key(kc, bt, 0, j, 1.5)
+    if mode == "dense":
+        out, lse, _, _ = run_dense(q, kc, bt, ld, SCALE, False, 1)
+        refs = dense_refs(q, kc, bt, ld, SCALE, False)
+    else:
+        out, lse = run_sparse(q, kc, bt, ld, idx, SCALE, mode == "fp8", 1)
+        refs = sparse_refs(q, kc, bt, ld, idx, SCALE, mode == "fp8")
+    assert float(refs[1][0, head]) > 120.0  # the planted key dominates that row
+    assert float(refs[1].sum() - refs[1][0, head]) < 20.0 * h_q  # and no other
+    assert_close(out, lse, *refs)
+
+
 # ---------------------------------------------------------------- sparse
 
 @pytest.mark.parametrize("name,fp8", [("sparse_bf16.npz", False), ("sparse_fp8.npz", True)])
