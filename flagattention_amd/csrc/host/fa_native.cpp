@@ -316,23 +316,44 @@ bool gqa_dtype(const at::Tensor& t) {
   return t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16;
 }
 
-// The split rule of gqa.py (choose_splits): rows = query rows per KV head, pairs = batch x KV
-// heads.
+// The split rule of gqa.py, whose comments say why its lines lie there; its constants have the
+// same names there, and tests/test_native_host.py compares the two rules.
+constexpr int64_t kRowsPerWg = 16;
+constexpr int64_t kMinSplitTokens = 256;
+constexpr int64_t kShortSplitTokens = 128;
+constexpr int64_t kMaxShortSplits = 64, kMaxShortSplitsSmallDim = 16;
+constexpr int64_t kMaxShortPartials = int64_t{1} << 21;
+constexpr int64_t kPrefillMinRows = 16;
+constexpr int64_t kPrefillRowsPerWg = 128;
+constexpr int64_t kPrefillUnsplitTokens = 512;
+constexpr int64_t kPrefillMaxPartials = int64_t{1} << 20;
+
+// rows = query rows per KV head, pairs = batch x KV heads.
 int64_t choose_splits(int64_t pairs, int64_t rows, int64_t rows_per_wg, int64_t d, int64_t max_len,
                       int64_t cus) {
   const int64_t base = pairs * cdiv(rows, rows_per_wg);
-  if (base >= cus || max_len <= 256) return 1;
-  const int64_t s = std::min(cdiv(2 * cus, base), cdiv(max_len, 256));
-  const int64_t few = std::min(cdiv(cus, base), cdiv(max_len, 128));
-  if (few > (d > 64 ? 64 : 16) || pairs * rows * few * d > (int64_t{1} << 21)) return s;
+  if (base >= cus || max_len <= kMinSplitTokens) return 1;
+  const int64_t s = std::min(cdiv(2 * cus, base), cdiv(max_len, kMinSplitTokens));
+  const int64_t few = std::min(cdiv(cus, base), cdiv(max_len, kShortSplitTokens));
+  if (few > (d > 64 ? kMaxShortSplits : kMaxShortSplitsSmallDim) ||
+      pairs * rows * few * d > kMaxShortPartials)
+    return s;
   return std::max(s, few);
 }
 
-// Whether a many-row call of few keys runs unsplit (gqa.py, prefill_unsplit).
+// Whether a many-row call of few keys runs unsplit.
 bool prefill_unsplit(int64_t pairs, int64_t rows, int64_t d, int64_t n, int64_t cus) {
-  if (n > 512) return false;
-  const int64_t few = std::min(cdiv(cus, pairs * cdiv(rows, 128)), cdiv(n, 128));
-  return n <= (d == 256 ? 256 : 384) || few < 3 || pairs * rows * few * d > (int64_t{1} << 20);
+  if (n > kPrefillUnsplitTokens) return false;
+  const int64_t few =
+      std::min(cdiv(cus, pairs * cdiv(rows, kPrefillRowsPerWg)), cdiv(n, kShortSplitTokens));
+  return n <= (d == 256 ? 256 : 384) || few < 3 || pairs * rows * few * d > kPrefillMaxPartials;
+}
+
+// Splits of a contiguous call.
+int64_t contiguous_splits(int64_t pairs, int64_t rows, int64_t d, int64_t n, int64_t cus) {
+  const bool many = (d == 64 || d == 128 || d == 256) && rows > kPrefillMinRows;
+  if (many && prefill_unsplit(pairs, rows, d, n, cus)) return 1;
+  return choose_splits(pairs, rows, many ? kPrefillRowsPerWg : kRowsPerWg, d, n, cus);
 }
 
 // whole 32-key tiles (gqa.py)
@@ -386,7 +407,7 @@ PyObject* paged(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int cus = cu_count(device.index());
     if (cus == 0) return none();
     split_tokens = whole_tiles(
-        cdiv(max_len, choose_splits(seqs * h_kv, h_q / h_kv, 16, d, max_len, cus)));
+        cdiv(max_len, choose_splits(seqs * h_kv, h_q / h_kv, kRowsPerWg, d, max_len, cus)));
   } else if (num_splits == 1) {
     split_tokens = max_len;
   } else {
@@ -461,12 +482,7 @@ PyObject* contiguous(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (k->device() != device || v->device() != device) return none();
   const int cus = cu_count(device.index());
   if (cus == 0) return none();
-  // the row counts and split rule of gqa.py
-  const int64_t rows = h_q / h_kv * m;
-  const bool many = (d == 64 || d == 128 || d == 256) && rows > 16;
-  int64_t s = many && prefill_unsplit(batch * h_kv, rows, d, n, cus)
-                  ? 1
-                  : choose_splits(batch * h_kv, rows, many ? 128 : 16, d, n, cus);
+  int64_t s = contiguous_splits(batch * h_kv, h_q / h_kv * m, d, n, cus);
   int64_t split_tokens = whole_tiles(cdiv(n, s));
   s = cdiv(n, split_tokens);
   if (s == 1) split_tokens = 1 << 30;
@@ -519,6 +535,18 @@ PyObject* contiguous(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Py_XDECREF(l);
   return both;
   END_HANDLE_TH_ERRORS
+}
+
+// split_counts(pairs, rows, d, n, cus): the split counts that the rule gives a paged and a
+// contiguous call (1 or more of each extent), for the comparison with gqa.py.
+PyObject* split_counts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  int64_t x[5];
+  if (nargs != 5) return none();
+  for (int i = 0; i < 5; ++i)
+    if (!to_int(args[i], &x[i]) || x[i] < 1) return none();
+  return Py_BuildValue(
+      "(LL)", static_cast<long long>(choose_splits(x[0], x[1], kRowsPerWg, x[2], x[3], x[4])),
+      static_cast<long long>(contiguous_splits(x[0], x[1], x[2], x[3], x[4])));
 }
 
 // ---- topk_indices(scores, cache_seqlens, topk, causal), result allocated here ----
@@ -608,7 +636,7 @@ PyObject* cache_write(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
    nullptr}
 PyMethodDef g_methods[] = {FA_METHOD(mla_metadata), FA_METHOD(mla_decode),   FA_METHOD(paged),
                            FA_METHOD(contiguous),   FA_METHOD(topk_indices), FA_METHOD(cache_write),
-                           {nullptr, nullptr, 0, nullptr}};
+                           FA_METHOD(split_counts), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, g_methods};
 
 }  // namespace

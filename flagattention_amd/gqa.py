@@ -46,6 +46,7 @@ MIN_SPLIT_TOKENS = 256
 # partial values (4 x 128 positions, 8 heads, 900 keys: 17.8 us in 4 splits, 21.2 in 8).
 SHORT_SPLIT_TOKENS = 128
 MAX_SHORT_SPLITS = 64
+MAX_SHORT_SPLITS_SMALL_DIM = 16
 MAX_SHORT_PARTIALS = 1 << 21
 # The many-row kernel (csrc/fa_prefill.h): head dims, rows per KV head above which the
 # library uses it for contiguous K/V, and its rows per work-group.
@@ -101,7 +102,7 @@ def choose_splits(batch: int, h_kv: int, rows_per_kv_head: int, max_len: int,
         return 1
     s = min(-(-2 * cu_count // base), -(-max_len // MIN_SPLIT_TOKENS))
     short = min(-(-cu_count // base), -(-max_len // SHORT_SPLIT_TOKENS))
-    if (short > (MAX_SHORT_SPLITS if head_dim > 64 else 16) or
+    if (short > (MAX_SHORT_SPLITS if head_dim > 64 else MAX_SHORT_SPLITS_SMALL_DIM) or
             batch * h_kv * rows_per_kv_head * short * head_dim > MAX_SHORT_PARTIALS):
         return s
     return max(s, short)
@@ -116,6 +117,16 @@ def prefill_unsplit(batch: int, h_kv: int, rows: int, n: int, cu_count: int,
     short = min(-(-cu_count // base), -(-n // SHORT_SPLIT_TOKENS))
     return (n <= (256 if head_dim == 256 else 384) or short < 3 or
             batch * h_kv * rows * short * head_dim > PREFILL_MAX_PARTIALS)
+
+
+def contiguous_splits(batch: int, h_kv: int, rows: int, n: int, cu_count: int,
+                      head_dim: int) -> int:
+    """Splits of a contiguous call (csrc/host/fa_native.cpp has the same rule)."""
+    many = head_dim in PREFILL_DIMS and rows > PREFILL_MIN_ROWS
+    if many and prefill_unsplit(batch, h_kv, rows, n, cu_count, head_dim):
+        return 1
+    return choose_splits(batch, h_kv, rows, n, cu_count,
+                         PREFILL_ROWS_PER_WG if many else ROWS_PER_WG, head_dim)
 
 
 def whole_tiles(tokens: int) -> int:
@@ -257,12 +268,7 @@ def _dense_decode(q, k, v, causal, sm_scale, want_lse):
     if o.stride(-1) != 1 or not _aligned(o, (0, 1, 2)):
         o = torch.empty(q.shape, dtype=q.dtype, device=device)
     lse = torch.empty((batch, h_q, m), dtype=torch.float32, device=device) if want_lse else None
-    rows = (h_q // h_kv) * m
-    many = d in PREFILL_DIMS and rows > PREFILL_MIN_ROWS
-    cus = _cu_count(device)
-    s = (1 if many and prefill_unsplit(batch, h_kv, rows, n, cus, d)
-         else choose_splits(batch, h_kv, rows, n, cus,
-                            PREFILL_ROWS_PER_WG if many else ROWS_PER_WG, d))
+    s = contiguous_splits(batch, h_kv, (h_q // h_kv) * m, n, _cu_count(device), d)
     split_tokens = whole_tiles(-(-n // s)) if n > 0 else 1
     s = max(1, -(-n // split_tokens)) if n > 0 else 1
     if s == 1:

@@ -29,6 +29,23 @@ def test_calls_without_gpu_tensors_are_left_to_python():
     assert fast.ABI_VERSION == _lib.ABI_VERSION
 
 
+@pytest.mark.parametrize("d", gqa.HEAD_DIMS)
+def test_split_rule_is_the_python_one(d):
+    """Every line of the split rule lies at the same place in both: the extents on each side of
+    it (key counts around the split lengths and their limits, row counts around a work-group's,
+    pairs up to a full chip)."""
+    fast = _lib.native()
+    lens = sorted({1, 5000, 8191, 8192, 8193, 70001} |
+                  {k * 128 + e for k in range(1, 17) for e in (0, 1)})
+    for cus in (64, 256, 304):
+        for pairs in (1, 2, 7, 8, 31, 32, 64, 100, 255, 256, 300):
+            for rows in (1, 8, 15, 16, 17, 40, 127, 128, 129, 400, 1500, 4096):
+                for n in lens:
+                    assert fast.split_counts(pairs, rows, d, n, cus) == (
+                        gqa.choose_splits(pairs, 1, rows, n, cus, head_dim=d),
+                        gqa.contiguous_splits(1, pairs, rows, n, cus, d)), (pairs, rows, n, cus)
+
+
 def _both(monkeypatch, call):
     """The call's results with and without the native path."""
     a = call()
@@ -115,14 +132,19 @@ def test_mla_matches_python_path(monkeypatch, mode, B, h, s_q, parts):
         kc = torch.randn((B * 16, 64, 1, 576), device="cuda").bfloat16()
     meta = lambda: flag_attn.get_mla_metadata(  # noqa: E731
         lens, s_q * h, 1, num_heads_q=h, topk=topk, num_sm_parts=parts)
+    assert _lib.native().mla_metadata(lens, s_q * h, 1, h, topk, parts) is not None
+    assert _lib.native().mla_metadata(lens.long(), s_q * h, 1, h, topk, parts) is None
     (md, ns), python = _both(monkeypatch, meta)
     _same((md, ns), python)
     assert md._fa_mla_sig == python[0]._fa_mla_sig and ns._fa_mla_sig == python[1]._fa_mla_sig
-    _same(*_both(monkeypatch, lambda: flag_attn.flash_mla_with_kvcache(
-        q, kc, bt, lens, 512, md, ns, None, mode == "dense", mode == "fp8", idx)))
+    args = (q, kc, bt, lens, 512, md, ns, None, mode == "dense", mode == "fp8", idx)
+    assert _lib.native().mla_decode(*args) is not None
+    assert _lib.native().mla_decode(q.float(), *args[1:]) is None
+    _same(*_both(monkeypatch, lambda: flag_attn.flash_mla_with_kvcache(*args)))
     with pytest.raises(mla.MLAArgumentError):  # metadata of another batch
         other, other_ns = flag_attn.get_mla_metadata(lens.repeat(2), s_q * h, 1, num_heads_q=h,
                                                      topk=topk)
+        assert _lib.native().mla_decode(*args[:5], other, *args[6:]) is None
         flag_attn.flash_mla_with_kvcache(q, kc, bt, lens, 512, other, ns, None, False,
                                          mode == "fp8", idx)
 
@@ -142,10 +164,15 @@ def test_write_and_topk_match_python_path(monkeypatch, fp8, slots):
         flag_attn.concat_and_cache_mla(kv, pe, cache, at, fp8)
         return cache
 
+    fresh = torch.zeros((2, 64, 1, row), dtype=dt, device="cuda")
+    assert _lib.native().cache_write(kv, pe, fresh, at, fp8) is True
+    assert _lib.native().cache_write(kv, pe, fresh, at.float(), fp8) is None
     _same(*_both(monkeypatch, write))
     for n, k in ((700, 64), (40000, 2048)):
         scores = torch.randn((2, 2, n), device="cuda")
         lens = torch.tensor([n, n // 2], dtype=torch.int32, device="cuda")
+        assert _lib.native().topk_indices(scores, lens, k, True) is not None
+        assert _lib.native().topk_indices(scores.half(), lens, k, True) is None
         _same(*_both(monkeypatch, lambda: flag_attn.topk_indices(scores, lens, k, True)))
 
 
