@@ -7,7 +7,9 @@
 // whose every split is empty (or that has no split at all) gets out = 0 and
 // lse = -inf, the convention of src/flag_attn/split_kv.py:161-164.
 //
-// One 64-lane wave per (sequence, query row); each lane owns 8 of the 512
+// Two kernels, chosen by combine_waves below: one 64-lane wave per (sequence,
+// query row), described here, or a work-group of four or eight waves per row
+// where the splits are many (mla_combine_wide_kernel).  Each lane owns 8 of the 512
 // value dims, so a bf16 partial row is one 16-byte load per lane (partials
 // are stored in bf16: the combine and the decode epilogue move half the
 // bytes, and the weighted sum is accumulated in fp32).  Up to 8 splits (the
@@ -184,7 +186,7 @@ void mla_combine_kernel(
 }
 
 // Many splits per sequence (a long context over few sequences): one work-group of kWideWaves
-// waves per row.  Wave w takes splits w, w + kWideWaves, ..., kWideBatch of them requested at
+// waves per row, bound by the latency of its loads.  Wave w takes splits w, w + kWideWaves, ..., kWideBatch of them requested at
 // once with their lse, and folds them against its own running max; the states are merged
 // through LDS.  The wave-per-row kernel walks them four at a time, three dependent round
 // trips each: 256 splits of 16 rows took 33.8 us there (a step of one 20,000-token sequence,
@@ -192,8 +194,11 @@ void mla_combine_kernel(
 constexpr int kWideBatch = 4;
 
 // Waves per row: 1 (the kernel above) for up to 8 splits a sequence, whose loads it issues at
-// once.  The split counts are device data; they are bounded by the parts a sequence can meet
-// and by its blocks.  Measured steps, 1 / 4 / 8 / 16 waves: 256 splits x 16 rows 47.1 / 30.4 /
+// once.  The split counts are device data; the rule goes by their average, the parts over the
+// sequences, and by the most that a sequence's blocks allow.  Where lengths differ a lot the
+// long sequences have more splits than the average, up to every part, and may run the kernel
+// above (32 sequences of 128 .. 65,536 tokens on 128 parts: 4 on average, up to 21; its combine
+// takes 10.4 us).  Measured steps, equal lengths, 1 / 4 / 8 / 16 waves: 256 splits x 16 rows 47.1 / 30.4 /
 // 24.9 / 23.6 us; 32 x 128 rows x 8 sequences 39.7 / 36.2 / 36.4 / 41.0; 16 x 16 rows x 16
 // sequences 24.2 / 22.3 / 21.7 / 23.1; 16 x 128 rows x 16 sequences 39.9 / 40.3 / 42.7 / 54.3
 // (enough rows to fill the chip: the extra waves only add work); 6 x 16 rows x 2 sequences
@@ -211,8 +216,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void mla_combine_wide_kernel(
     const bf16* __restrict__ o_accum, const float* __restrict__ lse_accum,
     const int32_t* __restrict__ num_splits, bf16* __restrict__ out, float* __restrict__ lse,
     int s_q, int h_q, int max_split) {
-  // states of the waves; the row pitch puts the 16 states of a dim in different banks
-  __shared__ float so[kWideWaves][kDv + 4];
+  __shared__ float so[kWideWaves][kDv];  // states of the waves
   __shared__ float sml[2][kWideWaves];
   const int rows = s_q * h_q;
   const int b = blockIdx.y, row = blockIdx.x;

@@ -836,7 +836,7 @@ __global__ __launch_bounds__(256) void gqa_combine_kernel(const fa_gqa_decode_ar
       for (int x = 0; x < 4; ++x) acc[v][x] *= f;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      if (lv[i] == ninf) continue;  // an empty split's values are not read
+      if (lv[i] == ninf) continue;  // an empty split's values are not used
       const float w = expf(lv[i] - mb);
       l += w;
 #pragma unroll

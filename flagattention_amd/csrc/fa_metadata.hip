@@ -138,7 +138,7 @@ struct Cuts<long long> {
   }
 };
 // 32-bit (W < 2^30, P <= 2^10): W = wq P + wr gives x_p = p wq + ceil(p wr / P), whose
-// quotient stays below 2^21, exact from a float estimate and one correction; the part of a
+// dividend stays below 2^21: exact from a float estimate and one correction; the part of a
 // position c comes from the float estimate c P / W (below 2^10, so within 1) and the cuts
 // beside it.
 template <>

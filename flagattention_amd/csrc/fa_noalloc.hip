@@ -11,7 +11,8 @@
 // array, so calls that overlap on one device (two streams, two threads) race
 // on it.  Nothing in it needs clearing between calls: each decode writes
 // every partial the combine then reads (the partials of the segments that
-// num_splits counts), and the row translation writes every gather row.
+// num_splits counts), and the row translation, where there is one (topk >
+// FA_MLA_FOLD_TOPK), writes every gather row.
 #include <mutex>
 
 #include "fa_common.h"
@@ -46,6 +47,8 @@ constexpr long long align256(long long x) { return (x + 255) / 256 * 256; }
 }  // namespace
 }  // namespace fa
 
+// Every sparse call is charged for its gather rows, also up to FA_MLA_FOLD_TOPK, where the
+// decode does without them: which calls fit does not depend on where the slots are translated.
 extern "C" int64_t fa_mla_noalloc_scratch_bytes(const fa_mla_decode_args* a, int32_t mode) {
   if (a == nullptr || a->batch < 1 || a->s_q < 1 || a->h_q < 1 || a->num_parts < 1) return -1;
   const long long segs = static_cast<long long>(a->batch) + a->num_parts;

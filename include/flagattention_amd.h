@@ -217,15 +217,17 @@ int fa_mla_topk_indices(const float* scores, int64_t stride_b, int64_t stride_t,
 int64_t fa_mla_topk_workspace_bytes(int32_t batch, int32_t s_q, int32_t len, int32_t topk);
 
 /*
- * Workspace bytes one fa_mla_decode_noalloc call with these arguments needs
- * (mode as below), or -1 if the shape fields are invalid.  A call fits when
- * this is <= FA_MLA_NOALLOC_SCRATCH_BYTES.
+ * Workspace bytes one fa_mla_decode_noalloc call with these arguments is
+ * charged for (mode as below; sparse modes always with their gather rows), or
+ * -1 if the shape fields are invalid.  A call fits when this is <=
+ * FA_MLA_NOALLOC_SCRATCH_BYTES.
  */
 int64_t fa_mla_noalloc_scratch_bytes(const fa_mla_decode_args* args, int32_t mode);
 
 /*
- * A whole decode step that allocates nothing: for sparse modes the row
- * translation, then the decode, then the combine -- the same kernels as
+ * A whole decode step that allocates nothing: for sparse modes with topk >
+ * FA_MLA_FOLD_TOPK the row translation, then the decode, then the combine --
+ * the same kernels as
  * fa_mla_sparse_rows + fa_mla_decode_dense / fa_mla_decode_sparse +
  * fa_mla_combine, with the split partials and gather rows kept in the
  * library's own device array (FA_MLA_NOALLOC_SCRATCH_BYTES per device)
