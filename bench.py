@@ -145,14 +145,14 @@ def build_inputs(spec, dev, copies):
 def algorithmic_work(spec, lens_cpu, indices) -> tuple:
     """HBM bytes and FLOPs one decode launch must move / compute: every KV row it
     attends to once, q in, out (or the split partial) and lse out, and the block-table
-    words (dense) or translated row ids (sparse) that address the rows; FLOPs of QK (576)
+    words (dense) or index slots (sparse) that address the rows; FLOPs of QK (576)
     and PV (512) per row and head."""
     b, s_q, h_q = spec["batch"], spec["s_q"], spec["h_q"]
     row_bytes = 656 if spec["fp8"] else 1152
     if spec["topk"]:
         n_valid = int((indices >= 0).sum())  # per (b, s) token lists
         kv_rows = n_valid
-        table = indices.numel() * 4  # the translated row ids
+        table = indices.numel() * 4  # the index slots
         flops_rows = n_valid  # each valid (b, s, token) pair meets h_q heads once
     else:
         kv_rows = int(lens_cpu.sum())
@@ -171,10 +171,22 @@ DECODE_SOURCES = ("flagattention_amd/csrc/fa_decode.hip",
                   "flagattention_amd/csrc/fa_mla_tile.h") + _SHARED
 KERNEL_SOURCES = {
     "mla_decode": DECODE_SOURCES,
-    "gqa_decode": ("flagattention_amd/csrc/fa_gqa_decode.hip",) + _SHARED,
+    "gqa_decode": ("flagattention_amd/csrc/fa_gqa_decode.hip",
+                   "flagattention_amd/csrc/fa_prefill.h") + _SHARED,
     "topk": ("flagattention_amd/csrc/fa_topk.hip",) + _SHARED,
     "kvcache": ("flagattention_amd/csrc/fa_kvcache.hip",) + _SHARED,
 }
+
+
+def step_kernels(spec) -> list:
+    """What one MLA step launches, in order: the scheduler metadata (in closed form for sparse
+    decode), the slot translation only for top-k lists longer than the decode translates itself,
+    the decode and the combine."""
+    from flagattention_amd.mla import FOLD_TOPK
+    topk = spec["topk"] or 0
+    return (["mla_metadata_uniform_kernel" if topk else "mla_metadata_kernel"] +
+            (["mla_sparse_rows_kernel"] if topk > FOLD_TOPK else []) +
+            ["mla_decode_kernel", "mla_combine_kernel"])
 
 
 def kernel_sources_sha(family: str = "mla_decode") -> str:
@@ -780,18 +792,13 @@ def run_mla(args) -> dict | None:
     if not args.no_cpu_baseline:
         cpu = cpu_baseline(spec, q, pools[0], tables[0], lens, indices)
 
-    # (a top-k list of up to FOLD_TOPK slots is translated to rows inside the decode)
-    from flagattention_amd.mla import FOLD_TOPK
-    step_kernels = ["mla_metadata_kernel"] + (
-        ["mla_sparse_rows_kernel"] if (spec["topk"] or 0) > FOLD_TOPK else [])
-    step_kernels += ["mla_decode_kernel", "mla_combine_kernel"]
     rec = {
         "metric": METRIC,
         "value": round(us_step, 2),
         "unit": "µs/step",
         # what one timed step launches, in order: the scheduler metadata is recomputed every
         # step (a model computes it once per forward pass and reuses it in every layer)
-        "step_kernels": step_kernels,
+        "step_kernels": step_kernels(spec),
         "n_gpus": 1,
         "steps": args.steps,
         "warmup": args.warmup,
