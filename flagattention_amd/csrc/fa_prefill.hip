@@ -20,7 +20,7 @@
 //     lanes away), so the row max is in-lane plus one lane swap, and the row sum stays
 //     in-lane until the end.  The reference that P is relative to follows each tile's
 //     maximum, down as well as up (kFall), and the accumulators are rescaled at every tile:
-//     the largest P of a tile is then exactly 1, and its rounding to 16 bits costs nothing.
+//     the largest P of a tile is then a power of two, and rounding it to 16 bits costs nothing.
 //     With one running maximum instead (rescaling only where some row has a new one) a long
 //     row has few such keys: 2% faster, but bf16 error against 64 bits 2.26e-3 instead of
 //     2.09e-3 at the first shape below, where the 16-row kernel (a reference per 32-key tile
@@ -58,13 +58,15 @@ constexpr int kPWaveRows = 32;
 static_assert(kPWaves * kPWaveRows == kPrefillRows, "rows per work-group");
 // A row's reference is the rounded product of its largest score and the scale; the fused
 // multiply-add of the exponents does not round that product, which leaves the largest
-// exponent at the rounding error instead of 0: up to 2^-15 for references below 2^10 (P still
-// rounds to 1), but +-32 at 2^30.  Past this reference the scores are scaled in a pass of their
-// own.
+// exponent at the rounding error instead of a whole number: up to 2^-15 for references below
+// 2^10 (P still rounds to a power of two), but +-32 at 2^30.  Past this reference the scores
+// are scaled in a pass of their own.
 constexpr float kFusedScale = 1024.f;
-// How far below a row's running maximum (log2 units) its reference may fall: the sums grow by
-// at most 2^4 over those of one running maximum.  Error at the first shape above 2.11e-3 at 2,
-// 2.090e-3 at 4 and at 8.
+// How far below a row's running maximum (log2 units) the maximum that P follows may fall.
+// Error at the first shape above 2.11e-3 at 2, 2.090e-3 at 4 and at 8.  In bf16 the reference
+// lies kFall above that maximum (the largest P of a tile is 2^-4, as exact as 1), so never
+// below the running one, and the sums of any finite V stay as far from overflow as with it.
+// fp16 keeps 1: its P would lose bits below 2^-14, and its V is at most 2^16.
 constexpr float kFall = 4.f;
 // Up to this many keys that a row sees on average, the 32-key halves of a 64-key tile take a
 // reference each.  bf16 error against 64 bits, 16-row kernel / tile / halves: 300 keys
@@ -314,7 +316,8 @@ __global__ __launch_bounds__(kPThreads, 2) void gqa_prefill_kernel(const fa_gqa_
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[tt][i]);
       mx = max_xor32(mx) * scale_log2;
       mrun = fmaxf(mrun, mx);
-      const float m_new = fmaxf(mx, mrun - kFall);
+      const float m_new =
+          __is_same(T, __bf16) ? fmaxf(mx + kFall, mrun) : fmaxf(mx, mrun - kFall);
       const float alpha = m_new == ninf ? 1.f : __builtin_amdgcn_exp2f(mref - m_new);
       lsum *= alpha;
       mref = m_new;

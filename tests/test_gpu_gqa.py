@@ -515,3 +515,19 @@ def test_empty_batch_or_query_is_the_librarys_argument_error(B, M, N):
         cache = torch.zeros((4, 2, 16, 64), dtype=torch.float16, device=DEV)
         with pytest.raises(RuntimeError, match="must be >= 1"):
             flag_attn.paged_attention(q[:, :, 0], cache, cache, lens, lens.new_zeros((0, 8)), 1.0, N)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("N", [300, 2100])  # references per half and per tile
+def test_flash_attention_many_rows_huge_values(D, N):
+    """One V row of the largest finite bf16 value, of any weight: the sums of a row never grow
+    past the weights' own, whatever the maxima of the tiles after it."""
+    need_gpu()
+    q, k, v = _splitkv_inputs(1, 4, 2, 40, N, D, torch.bfloat16, "BHTD", 1.0, D + N)
+    v[:, 0, 50], v[:, 1, 7] = torch.finfo(torch.bfloat16).min, torch.finfo(torch.bfloat16).max
+    o = flag_attn.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV)).cpu()
+    kd, vd = (x.double().repeat_interleave(2, dim=1) for x in (k, v))
+    p = torch.softmax(torch.matmul(q.double(), kd.transpose(2, 3).contiguous()) * D ** -0.5, dim=-1)
+    ref = torch.matmul(p, vd)
+    # P and out round to 8 bits (2^-9 each), the scores' own error is far below
+    assert bool(((o.double() - ref).abs() <= 2.0 ** -7 * ref.abs()).all())
