@@ -186,11 +186,11 @@ void mla_combine_kernel(
 }
 
 // Many splits per sequence (a long context over few sequences): one work-group of kWideWaves
-// waves per row, bound by the latency of its loads.  Wave w takes splits w, w + kWideWaves, ..., kWideBatch of them requested at
-// once with their lse, and folds them against its own running max; the states are merged
-// through LDS.  The wave-per-row kernel walks them four at a time, three dependent round
-// trips each: 256 splits of 16 rows took 33.8 us there (a step of one 20,000-token sequence,
-// 16 heads, 47.1 us), about 9 us here (24.9 us).
+// waves per row, bound by the latency of its loads.  Wave w takes splits w, w + kWideWaves,
+// ..., kWideBatch of them requested at once with their lse, and folds them against its own
+// running max; the states are merged through LDS.  The wave-per-row kernel walks them four at a
+// time, three dependent round trips each: 256 splits of 16 rows took 33.8 us there (a step of
+// one 20,000-token sequence, 16 heads, 47.1 us), about 9 us here (24.9 us).
 constexpr int kWideBatch = 4;
 
 // Waves per row: 1 (the kernel above) for up to 8 splits a sequence, whose loads it issues at
@@ -198,11 +198,11 @@ constexpr int kWideBatch = 4;
 // sequences, and by the most that a sequence's blocks allow.  Where lengths differ a lot the
 // long sequences have more splits than the average, up to every part, and may run the kernel
 // above (32 sequences of 128 .. 65,536 tokens on 128 parts: 4 on average, up to 21; its combine
-// takes 10.4 us).  Measured steps, equal lengths, 1 / 4 / 8 / 16 waves: 256 splits x 16 rows 47.1 / 30.4 /
-// 24.9 / 23.6 us; 32 x 128 rows x 8 sequences 39.7 / 36.2 / 36.4 / 41.0; 16 x 16 rows x 16
-// sequences 24.2 / 22.3 / 21.7 / 23.1; 16 x 128 rows x 16 sequences 39.9 / 40.3 / 42.7 / 54.3
-// (enough rows to fill the chip: the extra waves only add work); 6 x 16 rows x 2 sequences
-// 14.0 / 14.6 / 14.9 / 15.9.
+// takes 10.6 us).  Measured steps, equal lengths, 1 / 4 / 8 / 16 waves: 256 splits x 16 rows
+// 47.1 / 30.4 / 24.9 / 23.6 us; 32 x 128 rows x 8 sequences 39.7 / 36.2 / 36.4 / 41.0; 16 x 16
+// rows x 16 sequences 24.2 / 22.3 / 21.7 / 23.1; 16 x 128 rows x 16 sequences 39.9 / 40.3 /
+// 42.7 / 54.3 (enough rows to fill the chip: the extra waves only add work); 6 x 16 rows x 2
+// sequences 14.0 / 14.6 / 14.9 / 15.9.
 int combine_waves(const fa_mla_decode_args* a) {
   const long long parts = a->num_parts / a->batch;
   const long long blocks = a->topk > 0 ? cdiv(a->topk, kPage) : a->max_blocks_per_seq;

@@ -40,10 +40,10 @@ MIN_SPLIT_TOKENS = 256
 # Splits of one 32-key tile per wave where the launch is bound by the length of a work-group's
 # chain of tiles: 8 sequences of up to 1,000 tokens (32 heads of 4 KV heads, D = 128, paged)
 # 11.6 us a call in 4 splits, 10.5 in 8; one of 1,000 at D = 512 27.5 -> 17.7; 5 positions
-# x group 8 over 1,000 keys 11.6 -> 9.4.  Not once the CUs are full, and not where the combine
+# x group 8 over 1,000 keys 11.8 -> 9.4.  Not once the CUs are full, and not where the combine
 # would take back what they give: above 64 splits (16 up to head dim 64; 4 heads over 20,000
 # keys, D = 64: 8.6 us in 79 splits, 9.3 in 157; over 4,000 7.7 in 16, 7.9 in 32) or above 2^21
-# partial values (4 x 128 positions, 8 heads, 900 keys: 17.8 us in 4 splits, 21.2 in 8).
+# partial values (4 x 128 positions, 8 heads, 900 keys: 18.8 us in 4 splits, 21.6 in 8).
 SHORT_SPLIT_TOKENS = 128
 MAX_SHORT_SPLITS = 64
 MAX_SHORT_SPLITS_SMALL_DIM = 16
@@ -56,9 +56,9 @@ PREFILL_ROWS_PER_WG = 128
 # Up to 512 keys the many-row kernel splits only where at least 3 short splits leave at most
 # 2^20 partial values, and there from 385 keys (257 at head dim 256, whose tiles are half as
 # long): otherwise the second launch costs more than the keys it saves a work-group.  Per call,
-# unsplit / split: 5 positions x group 4 over 500 keys (8 KV heads, D = 128) 13.5 / 8.8 us, 4 x 8
-# over 300 at D = 256 21.3 / 12.6; but a 300-token prompt at D = 128 10.7 / 12.8, at D = 64 8.0 /
-# 10.3, and 100 x 4 over 400 keys (1.6 million partial values) 13.8 / 14.8.
+# unsplit / split: 5 positions x group 4 over 500 keys (8 KV heads, D = 128) 14.6 / 9.2 us, 4 x 8
+# over 300 at D = 256 20.5 / 12.3; but a 300-token prompt at D = 128 11.3 / 13.0, at D = 64 8.6 /
+# 10.5, and 100 x 4 over 400 keys (1.6 million partial values) 14.8 / 15.1.
 PREFILL_UNSPLIT_TOKENS = 512
 PREFILL_MAX_PARTIALS = 1 << 20
 
