@@ -334,7 +334,9 @@ int64_t choose_splits(int64_t pairs, int64_t rows, int64_t rows_per_wg, int64_t 
   const int64_t base = pairs * cdiv(rows, rows_per_wg);
   if (base >= cus || max_len <= kMinSplitTokens) return 1;
   const int64_t s = std::min(cdiv(2 * cus, base), cdiv(max_len, kMinSplitTokens));
-  const int64_t few = std::min(cdiv(cus, base), cdiv(max_len, kShortSplitTokens));
+  const bool one_wg_per_cu = rows_per_wg == kRowsPerWg && d >= 256;
+  const int64_t few =
+      std::min(one_wg_per_cu ? cus / base : cdiv(cus, base), cdiv(max_len, kShortSplitTokens));
   if (few > (d > 64 ? kMaxShortSplits : kMaxShortSplitsSmallDim) ||
       pairs * rows * few * d > kMaxShortPartials)
     return s;

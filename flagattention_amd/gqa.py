@@ -91,6 +91,13 @@ def _cu_count(device: torch.device) -> int:
     return _cu_counts[idx]
 
 
+def one_wg_per_cu(rows_per_wg: int, head_dim: int) -> bool:
+    """Whether the kernel's LDS leaves a CU one work-group: then short splits past one per CU
+    would run after all the others (60 KV heads, D = 256, 800 keys of 16 rows: 5 splits
+    37.0 us, 4 23.0)."""
+    return rows_per_wg == ROWS_PER_WG and head_dim >= 256
+
+
 def choose_splits(batch: int, h_kv: int, rows_per_kv_head: int, max_len: int,
                   cu_count: int, rows_per_wg: int = ROWS_PER_WG, head_dim: int = 128) -> int:
     """Split-KV count: none when batch x KV heads x row blocks already gives every CU a
@@ -101,7 +108,8 @@ def choose_splits(batch: int, h_kv: int, rows_per_kv_head: int, max_len: int,
     if base == 0 or base >= cu_count or max_len <= MIN_SPLIT_TOKENS:
         return 1
     s = min(-(-2 * cu_count // base), -(-max_len // MIN_SPLIT_TOKENS))
-    short = min(-(-cu_count // base), -(-max_len // SHORT_SPLIT_TOKENS))
+    per_cu = cu_count // base if one_wg_per_cu(rows_per_wg, head_dim) else -(-cu_count // base)
+    short = min(per_cu, -(-max_len // SHORT_SPLIT_TOKENS))
     if (short > (MAX_SHORT_SPLITS if head_dim > 64 else MAX_SHORT_SPLITS_SMALL_DIM) or
             batch * h_kv * rows_per_kv_head * short * head_dim > MAX_SHORT_PARTIALS):
         return s

@@ -46,6 +46,16 @@ def test_split_rule_is_the_python_one(d):
                         gqa.contiguous_splits(1, pairs, rows, n, cus, d)), (pairs, rows, n, cus)
 
 
+def test_short_splits_fit_the_chip_at_once():
+    """At head dims 256 and 512 a CU holds one work-group of the 16-row kernel: splits of under
+    256 keys must not leave some of them for a second turn."""
+    for d in (256, 512):
+        for pairs in range(1, 256):
+            for n in (257, 300, 520, 800, 1200, 3000):
+                s = gqa.choose_splits(1, pairs, 16, n, 256, head_dim=d)
+                assert s <= -(-n // gqa.MIN_SPLIT_TOKENS) or s * pairs <= 256, (d, pairs, n, s)
+
+
 def _both(monkeypatch, call):
     """The call's results with and without the native path."""
     a = call()
