@@ -441,6 +441,11 @@ bool prefill_takes(const fa_gqa_decode_args* a) {
   const long long rows = static_cast<long long>(a->h_q / a->h_kv) * a->m;
   if (a->block_table != nullptr || rows <= kPrefillMinRows) return false;
   if (a->d != 64 && a->d != 128 && a->d != 256) return false;
+  // few keys: the 16-row kernel, if it has few work-groups
+  const long long wg16 = static_cast<long long>(a->batch) * a->h_kv * ((rows + 15) / 16);
+  if (a->num_splits == 1 && !a->seqlens && a->n > few_keys_min(a->d) && a->n <= kFewKeysMax &&
+      wg16 <= few_keys_wgs(a->d))
+    return false;
   // 32-bit lane offsets inside a tile (64 rows)
   if (a->k_stride_t < 0 || a->v_stride_t < 0 || a->k_stride_t >= (1ll << 23) ||
       a->v_stride_t >= (1ll << 23))

@@ -49,7 +49,8 @@ MAX_SHORT_SPLITS = 64
 MAX_SHORT_SPLITS_SMALL_DIM = 16
 MAX_SHORT_PARTIALS = 1 << 21
 # The many-row kernel (csrc/fa_prefill.h): head dims, rows per KV head above which the
-# library uses it for contiguous K/V, and its rows per work-group.
+# library uses it for contiguous K/V (up to 256 keys, where nothing splits, not for all), and
+# its rows per work-group.
 PREFILL_DIMS = (64, 128, 256)
 PREFILL_MIN_ROWS = 16
 PREFILL_ROWS_PER_WG = 128

@@ -531,3 +531,23 @@ def test_flash_attention_many_rows_huge_values(D, N):
     ref = torch.matmul(p, vd)
     # P and out round to 8 bits (2^-9 each), the scores' own error is far below
     assert bool(((o.double() - ref).abs() <= 2.0 ** -7 * ref.abs()).all())
+
+
+@pytest.mark.parametrize("D, P, N, same", [
+    (64, 8, 64, False), (64, 8, 65, True), (64, 8, 256, True),  # one tile; the edges
+    (64, 64, 200, True), (64, 72, 200, False),   # 256 and 288 work-groups of 16 rows
+    (128, 4, 192, False), (128, 4, 193, True), (256, 4, 256, True),
+    (128, 5, 200, False), (256, 5, 200, False),  # 20 of them
+])
+def test_flash_attention_few_keys(D, P, N, same):
+    """Up to 256 keys: many rows run as blocks of 16 rows, with the bits of calls of 16 rows,
+    where that is the faster kernel; outside, the many-row kernel."""
+    need_gpu()
+    gen = torch.Generator(device=DEV).manual_seed(P + N)
+    q, k, v = (torch.randn((1, P, t, D), device=DEV, generator=gen).half() for t in (64, N, N))
+    o = flag_attn.flash_attention(q, k, v)
+    parts = torch.cat([flag_attn.flash_attention(c, k, v) for c in q.split(16, dim=2)], dim=2)
+    assert torch.equal(o, parts) == same
+    ref, _ = go.flash_attention_ref(q.cpu(), k.cpu(), v.cpu(), False, upcast=True)
+    low, _ = go.flash_attention_ref(q.cpu(), k.cpu(), v.cpu(), False, upcast=False)
+    assert_lowp_rule(o.cpu(), ref, low)
