@@ -298,7 +298,7 @@ int64_t fa_gqa_decode_args_size(void);
  * fa_gqa_combine.  Head dims 16, 32, 64, 128, 256, 512.  Contiguous K/V with more
  * than 16 query rows per KV head (group x m) at head dims 64, 128, 256 runs the
  * 128-row kernel of fa_prefill.hip (out must then have 16-byte aligned rows; if not,
- * the 16-row kernel runs).
+ * and for some calls of up to 256 keys, the 16-row kernel runs).
  * Replaces _paged_attn_kernel, src/flag_attn/paged.py:218-363 (paged) and
  * _fwd_split_kv_kernel, src/flag_attn/split_kv.py:28-174 (contiguous).
  */
