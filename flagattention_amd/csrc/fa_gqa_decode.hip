@@ -849,7 +849,7 @@ __global__ __launch_bounds__(256) void gqa_combine_kernel(const fa_gqa_decode_ar
   // them the partner's state is empty (2 splits of 130 rows, D = 16: 8.5 -> 7.7 us a call).
 #pragma unroll
   for (int off = 32; off >= kLanes; off >>= 1) {
-    if (kGroups == 1 && off >= kLanes * S) continue;  // uniform
+    if (kGroups == 1 && kPar > 2 && off >= kLanes * S) continue;  // uniform
     const float m2 = __shfl_xor(m, off), l2 = __shfl_xor(l, off);
     const float mn = fmaxf(m, m2);
     const float f1 = m == ninf ? 0.f : expf(m - mn), f2 = m2 == ninf ? 0.f : expf(m2 - mn);
